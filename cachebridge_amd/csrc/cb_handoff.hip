@@ -261,7 +261,7 @@ struct DevRows {
   int32_t index_kind;
   int32_t page_size;
   int32_t head_offset;
-  int32_t pad;
+  int32_t layers;
 };
 
 __device__ inline int64_t row_of(const DevRows& R, int t) {
@@ -324,6 +324,7 @@ __device__ inline gcptr layer_base(const DevRows& R, int kind, int layer) {
 struct MapArgs {
   const uint4* w;
   const float* bias;
+  const float* wscale;  // general kernel: inverse scale of each output dim's weights [job][D]
   const int4* jobs;
   const int32_t* pairs;
   const int32_t* unit_job;      // first job of each unit (jobs of a unit are consecutive)
@@ -344,6 +345,7 @@ struct MapArgs {
   int32_t chunk;
   int32_t ncls;
   int32_t cls_unit_begin[kMaxClasses];
+  int32_t cls_val_begin[kMaxClasses];  // general kernel: first values unit of each class
   int32_t cls_tok_first[kMaxClasses];
   int32_t cls_tok_count[kMaxClasses];
   int32_t cls_nchunks[kMaxClasses];
@@ -1787,191 +1789,779 @@ __global__ void pack_weights_kernel(const float* __restrict__ w, const float* __
 }
 
 // ---------------------------------------------------------------------------
-// Generic kernel: any even head_dim up to 512, any support, bf16 / fp16 /
-// fp32 K/V, computed in fp32 with FMAs (no split terms, no MFMA). It serves
-// the shapes and dtypes the MFMA kernels do not take; the configured
-// workloads never reach it.
+// General kernel: any even head_dim up to 512, any support, bf16 / fp16 /
+// fp32 K/V. It serves every shape and dtype that the streaming, support and
+// gen kernels do not take (head dims 256 and 96, fp16 pools, fp32 at 128).
 //
-// One workgroup of 256 threads per item (one job, a token range), 32-token
-// tiles. Per tile and support member k, the tile's source rows are gathered,
-// keys un-rotated (dims p and p + D/2 of a thread's pairs together), and the
-// fp32 values staged in LDS; each thread owns one output dim pair p, p + D/2
-// (threads_per_pair = 256 / (D/2) threads share a pair and split the
-// tokens) and accumulates sum_i x[t][i] * W[k*D + i][p] over the member's D
-// input dims. After the last member: + bias (the reference adds it after
-// the product), target RoPE on the pair, cast (round to nearest even),
-// store. Plan data for this kernel: W as fp32 [job][s*D][D] and the RoPE
-// tables in natural [theta][position][D/2] order.
+// A job is a [T x s*D] . [s*D x D] contraction; the plan keeps its maps in
+// fp32. The D/2 RoPE pairs (j, j + D/2) are padded to a multiple of 32 with
+// zero rows of W, so a job's input dims stream in chunks of 32 pairs (32
+// first-half dims, "part 0", and their partners, "part 1"), member after
+// member.
+//
+// Persistent workgroups map tiles of 16 tokens per wave of one job at a time.
+// Every chunk of a tile is gathered, un-rotated (keys) and split once, by all
+// waves, into MFMA operand order in one of two LDS buffers, while the waves
+// multiply the chunk in the other: one barrier per chunk. The chunks of
+// successive tiles form one stream, so a tile's gather, row indices and W
+// fragments are requested during the tile before it. Each wave owns 16 output
+// pairs (two row tiles: 16 first-half dims and their partners) of CT 16-token
+// column tiles, so nothing of W is shared between the waves of a tile and W
+// needs no LDS: a wave loads its own fp32 fragments a part ahead and splits
+// them in registers. 16-bit outputs leave through LDS, whole rows at a time.
+//
+// Products, all accumulated in fp32: bf16 splits both operands into three bf16
+// terms (24 bits; the products of terms i + j < 3: 6 for keys, 3 for values,
+// whose bf16 inputs are exact); fp16 into two fp16 terms of 11 bits each (3
+// and 2 products), with W scaled by a power of two per output dim at plan time
+// and keys by 1/2 (so that no finite input overflows); fp32 multiplies in
+// fp32, each part into accumulators of its own. The results are as close to
+// the 64-bit ones as those of fp32 fused multiply-adds (relative error at D
+// 256 bf16 1.658136e-3 with both, at D 128 fp16 2.07488e-4 and fp32 2.11e-7
+// with those, 2.07488e-4 and 1.57e-7 here; two bf16 terms gave 1.658142e-3).
+// An output that is not finite (an infinity or NaN in its source row) is
+// computed again term by term in fp32, because an infinity times the terms of
+// a weight need not keep its sign.
+//
+// Fragment layout (lane l: row or column l % 16, group g = l / 16): a part's
+// 32 dims are one MFMA k-step with lane group g holding dims 8g .. 8g + 7 (in
+// fp32, eight 4-dim k-steps: step e takes dim 8g + e of every group). The
+// accumulator register i of lane (col, g) is output dim 16 ng + 4g + i.
+//
+// Bound: latency and issue (MFMA 23-40% busy, HBM at 2-3 TB/s). Measured on
+// MI355X against a kernel of plain fp32 multiply-adds: 34x4 -> 48x8 at D 256
+// bf16 with windows, 2048 tokens, 16.5 -> 0.63 ms; 40x2 -> 64x2 at D 128 fp16,
+// 1000 tokens, 1.62 ms -> 69 us. What the parts cost at D 256 (removed one at
+// a time): products 16%, outputs 18%, gather and conversion 13%, W 5%.
 // ---------------------------------------------------------------------------
 
-constexpr int kAnyThreads = 256;
-constexpr int kAnyTile = 32;        // tokens per tile
+constexpr int kAnyTile = 32;        // granularity of tokens_per_workgroup
 constexpr int kAnyMaxDim = 512;
-constexpr int kAnyMaxTok = kAnyTile;  // tokens per thread at most (one thread per pair)
+constexpr int any_tokens(int nw) { return 16 * nw; }  // tokens per tile: four gathering threads each
+constexpr int kAnyRowBufs = 4;      // row tables: previous tile (epilogue) to the one after next
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+__host__ __device__ inline int any_chunks(int D) { return (D / 2 + 31) / 32; }   // chunks per support member
+__host__ __device__ inline int any_groups(int D) { return (D / 2 + 15) / 16; }   // 16-pair output groups
+// 16-byte units of one (chunk, part, output group): two row tiles x two 4-dim halves x 64 lanes.
+constexpr int kAnyFragU4 = 2 * 2 * kWave;
+// Float offset of W[member dim i][output o] of a job in the packed maps.
+__host__ __device__ inline int64_t any_w_offset(int D, int member, int i, int o) {
+  const int half = D / 2, part = i >= half, jp = part ? i - half : i;
+  const int tile = o >= half, op = tile ? o - half : o;
+  const int64_t stage = (static_cast<int64_t>(member) * any_chunks(D) + jp / 32) * 2 + part;
+  const int lane = (op & 15) + 16 * ((jp & 31) >> 3), e = jp & 7;
+  return (((stage * any_groups(D) + op / 16) * 2 + tile) * 2 + (e >> 2)) * (kWave * 4) + lane * 4 + (e & 3);
+}
 
 template <typename IO>
 struct AnyIO;
 template <>
 struct AnyIO<uint16_t> {  // bf16
+  using Frag = bf16x8;
+  static constexpr int kTerms = 3;
+  static constexpr float kKeyScale = 1.f;
+  static constexpr bool kScaled = false;
   static __device__ float get(const CB_GLOBAL uint16_t* p) { return bf2f(*p); }
-  static __device__ void put(CB_GLOBAL uint16_t* p, float v) { *p = f2bf(v); }
+  static __device__ uint16_t put(float v) { return f2bf(v); }
+  static __device__ uint32_t pack(float a, float b) { return pack_bf16(a, b); }
+  static __device__ float lo(uint32_t w) { return lo_bf(w); }
+  static __device__ float hi(uint32_t w) { return hi_bf(w); }
+  static __device__ f32x4 mul(const Frag& a, const Frag& b, const f32x4& c) { return mfma(a, b, c); }
 };
 template <>
 struct AnyIO<_Float16> {
+  using Frag = f16x8;
+  static constexpr int kTerms = 2;
+  static constexpr float kKeyScale = 0.5f;
+  static constexpr bool kScaled = true;  // weights scaled per output dim
   static __device__ float get(const CB_GLOBAL _Float16* p) { return static_cast<float>(*p); }
-  static __device__ void put(CB_GLOBAL _Float16* p, float v) { *p = static_cast<_Float16>(v); }
+  static __device__ _Float16 put(float v) { return static_cast<_Float16>(v); }
+  static __device__ uint32_t pack(float a, float b) {
+    const f16x2 h = {static_cast<_Float16>(a), static_cast<_Float16>(b)};
+    return __builtin_bit_cast(uint32_t, h);
+  }
+  static __device__ float lo(uint32_t w) { return static_cast<float>(__builtin_bit_cast(f16x2, w)[0]); }
+  static __device__ float hi(uint32_t w) { return static_cast<float>(__builtin_bit_cast(f16x2, w)[1]); }
+  static __device__ f32x4 mul(const Frag& a, const Frag& b, const f32x4& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
 };
 template <>
 struct AnyIO<float> {
+  static constexpr int kTerms = 2;  // (4-dim halves of a fragment)
+  static constexpr float kKeyScale = 1.f;
+  static constexpr bool kScaled = false;
   static __device__ float get(const CB_GLOBAL float* p) { return *p; }
-  static __device__ void put(CB_GLOBAL float* p, float v) { *p = v; }
+  static __device__ float put(float v) { return v; }
 };
 
+// Eight values as terms of the 16-bit type: each the rounded rest of those
+// before it, element pairs packed.
 template <typename IO>
-__global__ __launch_bounds__(kAnyThreads) void map_install_any_kernel(MapArgs a, int D) {
-#pragma clang fp contract(off)
-  __shared__ float xs[kAnyTile][kAnyMaxDim];
-  __shared__ int64_t trow[kAnyTile];
-  __shared__ int64_t srow[kAnyTile];  // source row, -1: zero source values
-  __shared__ int32_t tpos[kAnyTile];
-  Work wk;
-  if (!decode_work(a, &wk)) return;
-  const int S = a.support;
-  const int half = D / 2;
-  const int job = wk.job;
-  const int* jm = reinterpret_cast<const int*>(a.jobs + job);
-  const int mx = cload(jm), meta_y = cload(jm + 1);
-  const int kind = meta_y & 0xff;
-  const bool is_k = kind == CB_KIND_K;
-  const int sth = (meta_y >> 16) & 0xff, tth = (meta_y >> 24) & 0xff;
-  const int64_t eb = sizeof(IO);
-  // Un-rotation tables cos/m, sin/m and rotation tables, natural order.
-  const CB_GLOBAL float* ucos = gtab(a.ucos_tab) + sth * a.theta_stride;
-  const CB_GLOBAL float* usin = gtab(a.usin_tab) + sth * a.theta_stride;
-  const CB_GLOBAL float* rcos = gtab(a.cos_tab) + tth * a.theta_stride;
-  const CB_GLOBAL float* rsin = gtab(a.sin_tab) + tth * a.theta_stride;
-  gptr tbase = const_cast<gptr>(layer_base(a.tgt, kind, mx & 0xffff)) +
-               static_cast<int64_t>((mx >> 16) - a.tgt.head_offset) * D * eb;
-  const CB_GLOBAL float* W = gtab(reinterpret_cast<const float*>(a.w)) + static_cast<int64_t>(job) * S * D * D;
-  const CB_GLOBAL float* bias = gtab(a.bias) + static_cast<int64_t>(job) * D;
-  // This thread's dim pair and tokens.
-  const int tpp = max(1, kAnyThreads / half);       // threads per pair
-  const int p = threadIdx.x / tpp, sub = threadIdx.x % tpp;
-  const bool active = p < half;
-  const int toks = (kAnyTile + tpp - 1) / tpp;      // tokens per thread
-  int errbits = 0;
+__device__ __attribute__((always_inline)) inline void any_split(const float (&v)[8], uint32_t (&h)[AnyIO<IO>::kTerms][4]) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float a = v[2 * e], b = v[2 * e + 1];
+#pragma unroll
+    for (int t = 0; t < AnyIO<IO>::kTerms; ++t) {
+      h[t][e] = AnyIO<IO>::pack(a, b);
+      a = a - AnyIO<IO>::lo(h[t][e]);
+      b = b - AnyIO<IO>::hi(h[t][e]);
+    }
+  }
+}
 
-  for (int lo = wk.tok_lo; lo < wk.tok_hi; lo += kAnyTile) {
-    const int n = min(kAnyTile, wk.tok_hi - lo);
-    __syncthreads();  // the previous tile's LDS reads are done
-    if (threadIdx.x < kAnyTile) {
-      const int t = threadIdx.x;
-      const int tk = lo + min(t, n - 1);
-      const int64_t s = row_of(a.src, tk), d = row_of(a.tgt, tk);
-      const bool live = t < n;
-      const bool sok = s >= 0 && s < a.src.rows, dok = d >= 0 && d < a.tgt.rows;
-      if (live) errbits |= (sok ? 0 : 1) | (dok ? 0 : 2);
-      // A token whose source row is out of range writes nothing.
-      trow[t] = live && sok && dok ? d : -1;
-      srow[t] = live && sok ? s : -1;
-      tpos[t] = position_of(a, tk);
-    }
-    float acc[kAnyMaxTok][2];
+// Eight consecutive elements of a source row as raw words: dims [j, j + 8) of
+// a half-row, zero from `valid` on. WIDE: whole groups at 16-byte addresses.
+template <typename IO, bool WIDE>
+__device__ __attribute__((always_inline)) inline void any_load8(gcptr p, int valid, uint32_t (&out)[2 * sizeof(IO)]) {
+  if constexpr (WIDE) {
 #pragma unroll
-    for (int m = 0; m < kAnyMaxTok; ++m) acc[m][0] = acc[m][1] = 0.f;
+    for (int u = 0; u < static_cast<int>(sizeof(IO)) / 2; ++u) {
+      const uint4 v = gload<uint4>(p + 16 * u);
+      out[4 * u] = v.x; out[4 * u + 1] = v.y; out[4 * u + 2] = v.z; out[4 * u + 3] = v.w;
+    }
+  } else if constexpr (sizeof(IO) == 4) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out[e] = e < valid ? gload<uint32_t>(p + 4 * e) : 0u;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t a = 2 * e < valid ? gload<uint16_t>(p + 4 * e) : 0u;
+      const uint32_t b = 2 * e + 1 < valid ? gload<uint16_t>(p + 4 * e + 2) : 0u;
+      out[e] = a | (b << 16);
+    }
+  }
+}
+
+// Row table of one tile: source row byte offsets (-1: zeros), target rows
+// (-1: nothing is written) and positions.
+template <int TT>
+struct AnyRows {
+  int64_t src[TT], tgt[TT];
+  int32_t pos[TT];
+};
+
+// 16-bit outputs of a tile are staged in the X buffer that the tile's last
+// chunk leaves free: bytes of a token (NGW groups of 16 dims, two halves,
+// padded against bank conflicts) and size of a buffer, in 16-byte units.
+constexpr int any_stage_row(int nw, int ngw) { return ngw * 64 + (nw == 8 ? 32 : 16); }
+constexpr int any_buf_u4(int nw, int ngw, int planes, bool f32) {
+  const int tt = any_tokens(nw), x = planes * 2 * 4 * tt, st = tt * any_stage_row(nw, ngw) / 16;
+  return !f32 && st > x ? st : x;
+}
+
+// Tiles of the launch. The jobs of a window class are its keys, then its
+// values; the tiles of each run in blocks of kAnyJobs jobs, token tile by token
+// tile (jobs sorted together share source rows, and the tiles that run at one
+// time share their W in L2). XCD x takes the eighth x of every kind's tiles, so
+// that all XCDs get the same mix of keys and the cheaper values, and its
+// workgroups take them in turn.
+constexpr int kAnyJobs = 8;
+struct AnyTile {
+  int job, lo, hi;
+};
+// The tiles of one kind of one class that XCD x runs; `seg` counts them, class
+// by class, keys then values.
+struct AnySegment {
+  int begin, count;  // tiles [begin, begin + count) of the segment are this XCD's
+  int u0, nu, nch, first, end;
+};
+__device__ inline bool any_segment(const MapArgs& a, int x, int seg, AnySegment* g) {
+  const int c = seg >> 1;
+  if (c >= a.ncls) return false;
+  g->nch = a.cls_tok_count[c] > 0 ? a.cls_nchunks[c] : 0;
+  g->u0 = seg & 1 ? a.cls_val_begin[c] : a.cls_unit_begin[c];
+  g->nu = (seg & 1 ? a.cls_unit_end[c] : a.cls_val_begin[c]) - g->u0;
+  g->first = a.cls_tok_first[c];
+  g->end = g->first + a.cls_tok_count[c];
+  const int n = g->nu * g->nch;
+  g->begin = n / 8 * x + n % 8 * x / 8;
+  g->count = n / 8 * (x + 1) + n % 8 * (x + 1) / 8 - g->begin;
+  return true;
+}
+__device__ inline AnyTile any_tile(const MapArgs& a, const AnySegment& g, int p) {
+  const int idx = g.begin + p, blk = idx / (kAnyJobs * g.nch), r = idx - blk * kAnyJobs * g.nch;
+  const int gj = min(kAnyJobs, g.nu - blk * kAnyJobs);
+  const int tile = gj == kAnyJobs ? r / kAnyJobs : r / gj;
+  AnyTile t;
+  t.job = g.u0 + blk * kAnyJobs + r - tile * gj;  // units are single jobs, in job order
+  t.lo = g.first + tile * a.chunk;
+  t.hi = min(t.lo + a.chunk, g.end);
+  return t;
+}
+
+// Whether 16-byte accesses may be used: whole 8-dim groups and aligned layer
+// bases, which only the device can see where a side gives per-layer pointers
+// (one lane per pointer).
+__device__ inline bool any_wide(const MapArgs& a, int D) {
+  uint64_t bits = 0;
+#pragma unroll
+  for (int side = 0; side < 2; ++side) {
+    const DevRows& r = side ? a.tgt : a.src;
+    bits |= r.row_stride_b;
+    if (!r.k_layers) bits |= reinterpret_cast<uint64_t>(r.k_base) | reinterpret_cast<uint64_t>(r.v_base) | r.layer_stride_b;
+    for (int l = threadIdx.x & (kWave - 1); r.k_layers && l < r.layers; l += kWave)
+      bits |= reinterpret_cast<uint64_t>(r.k_layers[l]) | reinterpret_cast<uint64_t>(r.v_layers[l]);
+  }
+  return D % 16 == 0 && __builtin_amdgcn_ballot_w64((bits & 15) != 0) == 0;
+}
+
+// This workgroup's tiles of the segment: positions p, p + nwg, ... below its
+// count (at least one).
+// Output groups [NGW * blockIdx.y, + NGW) of each job, NGW = NW * 16 * CT / 128.
+template <typename IO, int NW, int CT, bool IS_K, bool WIDE>
+__device__ __attribute__((always_inline)) inline void any_run(const MapArgs& a, int D, const AnySegment& sg, int p, int nwg,
+                                                              uint4* xs, AnyRows<any_tokens(NW)>* tab) {
+#pragma clang fp contract(off)
+  constexpr bool F32 = sizeof(IO) == 4;
+  constexpr int WT = AnyIO<IO>::kTerms;             // terms of a weight (and of an un-rotated key)
+  constexpr int XP = F32 || IS_K ? WT : 1;          // planes per input: terms, or 4-dim halves (fp32)
+  constexpr int TT = any_tokens(NW);
+  constexpr int NGW = NW * 16 * CT / TT;            // output groups of the workgroup
+  constexpr int kPlane = TT * 4;                    // 16-byte units of one plane and part of a chunk
+  constexpr int RW = 2 * sizeof(IO);                // raw words of 8 elements
+  constexpr int kBuf = any_buf_u4(NW, NGW, WT, F32);    // uint4 per buffer; X: [plane][part][column tile][lane]
+  constexpr bool STAGED = WIDE && !F32;             // outputs leave through LDS, whole rows at a time
+  constexpr int kRowB = any_stage_row(NW, NGW);     // bytes of a staged token: both halves of the workgroup's dims
+  constexpr int kind = IS_K ? CB_KIND_K : CB_KIND_V;
+  constexpr int64_t eb = sizeof(IO);
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int g = lane >> 4, col = lane & 15;
+  const int half = D >> 1, Q = any_chunks(D), NG = any_groups(D), S = a.support, NC = S * Q, HP = Q * 32;
+  // This wave's outputs: pair group ng of token columns [64 or 128 wide] mg.
+  const int ng = static_cast<int>(blockIdx.y) * NGW + wave % NGW;
+  const int mg = wave / NGW;
+  const bool busy = ng < NG;  // waves past the last group only gather
+  // The current tile, the one after it (`next`, if `more`) and the one after
+  // that (the last tile again where there is none).
+  AnyTile cur = any_tile(a, sg, p);
+  auto advance = [&](AnyTile& t) __attribute__((always_inline)) {
+    p += nwg;
+    if (p >= sg.count) return false;
+    t = any_tile(a, sg, p);
+    return true;
+  };
+  AnyTile next = cur, then;
+  bool more, more2;
+  const int64_t wstage = static_cast<int64_t>(NG) * kAnyFragU4 * 16;
+
+  // Gathering: four threads per token, each one 8-dim group of both parts.
+  const int c4 = threadIdx.x & 3, gt = threadIdx.x >> 2;
+  int errbits = 0;
+  // Row table of the tile at lo: the index words are requested (by every
+  // thread, so that no branch surrounds the loads) a tile's products before
+  // they are resolved into LDS.
+  const int rt = threadIdx.x & (TT - 1);
+  const CB_GLOBAL uint32_t* spare = reinterpret_cast<const CB_GLOBAL uint32_t*>(as_global(a.sink));
+  uint2 fs, fd;
+  uint32_t fp;
+  auto fetch_rows = [&](const AnyTile& t) __attribute__((always_inline)) {
+    const int tk = min(t.lo + rt, t.hi - 1);
+    fs = row_fetch(a.src, tk, spare);
+    fd = row_fetch(a.tgt, tk, spare);
+    fp = *(a.pos ? reinterpret_cast<const CB_GLOBAL uint32_t*>(as_global(a.pos)) + tk : spare);
+  };
+  auto finish_rows = [&](const AnyTile& t, AnyRows<TT>& r, bool use) __attribute__((always_inline)) {
+    if (threadIdx.x >= TT || !use) return;
+    const int tk = min(t.lo + rt, t.hi - 1);
+    const bool live = t.lo + rt < t.hi;
+    const int64_t s = row_finish(a.src, tk, fs), d = row_finish(a.tgt, tk, fd);
+    const bool sok = s >= 0 && s < a.src.rows, dok = d >= 0 && d < a.tgt.rows;
+    if (live) errbits |= (sok ? 0 : 1) | (dok ? 0 : 2);
+    // A token whose source row is out of range writes nothing.
+    r.src[rt] = live && sok ? s * a.src.row_stride_b : -1;
+    r.tgt[rt] = live && sok && dok ? d : -1;
+    r.pos[rt] = a.pos ? static_cast<int32_t>(fp) : a.position_start + tk;
+  };
+
+  uint32_t raw[2][RW];
+  f32x4 uc[2], us[2];
+  gcptr zrow = as_global(a.zero);
+  // The chunk to gather next: member lk, pairs 32 lq .. of source head lbase
+  // (looked up when the chunk before it has been requested, so that no
+  // request waits for the job tables), un-rotation tables at utab.
+  int lk = 0, lq = 0;
+  auto head_base = [&](int job, int k) __attribute__((always_inline)) {
+    const int pr = cload(a.pairs + static_cast<int64_t>(job) * S + k);
+    return layer_base(a.src, kind, pr & 0xffff) + static_cast<int64_t>((pr >> 16) - a.src.head_offset) * D * eb;
+  };
+  auto thetas = [&](int job) __attribute__((always_inline)) {
+    return cload(reinterpret_cast<const int*>(a.jobs + job) + 1) >> 16;
+  };
+  gcptr lbase = head_base(cur.job, 0);
+  int64_t utab = (thetas(cur.job) & 0xff) * a.theta_stride;
+  auto load_raw = [&](const AnyRows<TT>& r) __attribute__((always_inline)) {
+    const int j = 32 * lq + 8 * c4;
+    const int valid = min(max(half - j, 0), 8);
+    const int64_t so = r.src[gt];
+    const bool ok = so >= 0 && valid > 0;
+    gcptr p = ok ? lbase + so + j * eb : zrow;
+    any_load8<IO, WIDE>(p, ok ? valid : 0, raw[0]);
+    any_load8<IO, WIDE>(ok ? p + half * eb : zrow, ok ? valid : 0, raw[1]);
+  };
+  // Its un-rotation values; then on to the chunk after it.
+  auto load_tab = [&](const AnyRows<TT>& r, int job_then) __attribute__((always_inline)) {
+    if constexpr (IS_K) {
+      const int64_t at = utab + static_cast<int64_t>(r.pos[gt]) * HP + 32 * lq + 8 * c4;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        uc[u] = gload<f32x4>((gcptr)(gtab(a.ucos_tab) + at + 4 * u));
+        us[u] = gload<f32x4>((gcptr)(gtab(a.usin_tab) + at + 4 * u));
+      }
+    }
+    lq = lq + 1 == Q ? 0 : lq + 1;
+    lk = lq ? lk : lk + 1 == S ? 0 : lk + 1;
+    if (lq == 0) {
+      lbase = head_base(job_then, lk);
+      if constexpr (IS_K) utab = (thetas(job_then) & 0xff) * a.theta_stride;
+    }
+  };
+  // Un-rotate and split the raw chunk into X buffer `x`.
+  auto convert = [&](uint4* x) __attribute__((always_inline)) {
+    auto put = [&](int plane, int part, uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3) __attribute__((always_inline)) {
+      x[(plane * 2 + part) * kPlane + (gt >> 4) * kWave + 16 * c4 + (gt & 15)] = make_uint4(w0, w1, w2, w3);
+    };
+    if constexpr (!IS_K) {
+#pragma unroll
+      for (int part = 0; part < 2; ++part)
+#pragma unroll
+        for (int pl = 0; pl < XP; ++pl)
+          put(pl, part, raw[part][4 * pl], raw[part][4 * pl + 1], raw[part][4 * pl + 2], raw[part][4 * pl + 3]);
+    } else {
+      float k1[8], k2[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float x1, x2;
+        if constexpr (F32) {
+          x1 = __uint_as_float(raw[0][e]);
+          x2 = __uint_as_float(raw[1][e]);
+        } else {
+          x1 = e & 1 ? AnyIO<IO>::hi(raw[0][e >> 1]) : AnyIO<IO>::lo(raw[0][e >> 1]);
+          x2 = e & 1 ? AnyIO<IO>::hi(raw[1][e >> 1]) : AnyIO<IO>::lo(raw[1][e >> 1]);
+        }
+        const float c = uc[e >> 2][e & 3], s = us[e >> 2][e & 3];
+        k1[e] = __builtin_fmaf(x1, c, x2 * s);
+        k2[e] = __builtin_fmaf(x2, c, -(x1 * s));
+        k1[e] *= AnyIO<IO>::kKeyScale;
+        k2[e] *= AnyIO<IO>::kKeyScale;
+      }
+      if constexpr (F32) {
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl) {
+          put(pl, 0, __float_as_uint(k1[4 * pl]), __float_as_uint(k1[4 * pl + 1]), __float_as_uint(k1[4 * pl + 2]), __float_as_uint(k1[4 * pl + 3]));
+          put(pl, 1, __float_as_uint(k2[4 * pl]), __float_as_uint(k2[4 * pl + 1]), __float_as_uint(k2[4 * pl + 2]), __float_as_uint(k2[4 * pl + 3]));
+        }
+      } else {
+        uint32_t h[2][WT][4];  // [part][term][element pair]
+        any_split<IO>(k1, h[0]);
+        any_split<IO>(k2, h[1]);
+#pragma unroll
+        for (int pl = 0; pl < XP; ++pl)
+#pragma unroll
+          for (int part = 0; part < 2; ++part) put(pl, part, h[part][pl][0], h[part][pl][1], h[part][pl][2], h[part][pl][3]);
+      }
+    }
+  };
+
+  f32x4 acc[2][CT];
+  f32x4 acc_b[2][F32 ? CT : 1];  // fp32: the products of part 1 (shorter sums)
+  f32x4 wr[2][2][2];  // fp32 W fragments [part][row tile][4-dim half]
+  auto load_w = [&](int job, int c, auto partc) __attribute__((always_inline)) {
+    constexpr int part = decltype(partc)::value;
+    gcptr p = as_global(a.w) + (static_cast<int64_t>(job) * NC * 2 + 2 * c + part) * wstage +
+              (min(ng, NG - 1) * (kAnyFragU4 * 16) + lane * 16);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) wr[part][t][u] = gload<f32x4>(p + (2 * t + u) * (kWave * 16));
+  };
+  // Products of one part of the chunk in `x` with the wave's first N column
+  // tiles. Straight-line code for a few N: branches between the tiles would
+  // cost 60 registers (copies of the accumulators where they join).
+  auto multiply_tiles = [&](const uint4* x, auto partc, auto nc) __attribute__((always_inline)) {
+    constexpr int part = decltype(partc)::value;
+    constexpr int N = decltype(nc)::value;
+    // A fragment is 1 KB in lane order: the only layout whose 16-byte reads
+    // found no bank conflicts (a padded [dim group][token] one lost half the
+    // LDS cycles to them; its writes had none, these have).
+    const uint4* xp = x + part * kPlane + mg * CT * kWave + lane;
+    if constexpr (F32) {
+#pragma unroll
+      for (int ct = 0; ct < N; ++ct) {
+        float xv[8];
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl) {
+          const uint4 v = xp[pl * 2 * kPlane + ct * kWave];
+          xv[4 * pl] = __uint_as_float(v.x); xv[4 * pl + 1] = __uint_as_float(v.y);
+          xv[4 * pl + 2] = __uint_as_float(v.z); xv[4 * pl + 3] = __uint_as_float(v.w);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+            (part ? acc_b : acc)[t][ct] =
+                __builtin_amdgcn_mfma_f32_16x16x4f32(wr[part][t][e >> 2][e & 3], xv[e], (part ? acc_b : acc)[t][ct], 0, 0, 0);
+        if (ct & 1) __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      typename AnyIO<IO>::Frag wf[2][WT];  // [row tile][term]
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const f32x4 w0 = wr[part][t][0], w1 = wr[part][t][1];
+        const float w[8] = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3]};
+        uint32_t h[WT][4];
+        any_split<IO>(w, h);
+#pragma unroll
+        for (int p = 0; p < WT; ++p)
+          wf[t][p] = __builtin_bit_cast(typename AnyIO<IO>::Frag, make_uint4(h[p][0], h[p][1], h[p][2], h[p][3]));
+      }
+      // The next column tile's inputs are read during this one's products
+      // (where its three planes leave the registers for it: not with CT 8).
+      constexpr int NB = XP * CT > 16 ? 1 : 2;
+      typename AnyIO<IO>::Frag xf[NB][XP];
+      auto read_x = [&](int ct) __attribute__((always_inline)) {
+#pragma unroll
+        for (int pl = 0; pl < XP; ++pl)
+          xf[ct % NB][pl] = __builtin_bit_cast(typename AnyIO<IO>::Frag, xp[pl * 2 * kPlane + ct * kWave]);
+      };
+      read_x(0);
+#pragma unroll
+      for (int ct = 0; ct < N; ++ct) {
+        if (NB == 2 && ct + 1 < N) read_x(ct + 1);
+        if (NB == 1 && ct > 0) read_x(ct);
+        for_products<XP, WT>([&](int i, int j) {
+#pragma unroll
+          for (int t = 0; t < 2; ++t) acc[t][ct] = AnyIO<IO>::mul(wf[t][j], xf[ct % NB][i], acc[t][ct]);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  auto multiply = [&](const uint4* x, auto partc, int nct) __attribute__((always_inline)) {
+    if (nct > CT / 2) multiply_tiles(x, partc, std::integral_constant<int, CT>{});
+    else if (nct > CT / 4) multiply_tiles(x, partc, std::integral_constant<int, CT / 2>{});
+    else if (nct > 0) multiply_tiles(x, partc, std::integral_constant<int, (CT + 3) / 4>{});
+  };
+
+  // Output pairs of this lane: 16 ng + 4g + i. The epilogue reads it through
+  // `hide`, so that nothing it derives stays in registers over the main loop.
+  const int jo_ = 16 * min(ng, NG - 1) + 4 * g;
+  auto hide = [](int v) __attribute__((always_inline)) {
+    asm volatile("" : "+v"(v));
+    return v;
+  };
+  auto out_values = [&](const float* p, int job, int jo, float (&v)[2][4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const CB_GLOBAL float* q = gtab(p) + static_cast<int64_t>(job) * D + t * half;
+      if constexpr (WIDE) {
+        const f32x4 w = gload<f32x4>((gcptr)(q + min(jo, half - 4)));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[t][i] = w[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[t][i] = q[min(jo + i, half - 1)];
+      }
+    }
+  };
+
+  // y of output pairs jo + i for one token, term by term in fp32 (rare: only
+  // where the split sum is not finite).
+  auto slow = [&](int tk, int jo, const float (&inv)[2][4], float (&y)[2][4]) __attribute__((always_inline)) {
+    const int job = cur.job;
+    const int64_t ro = row_of(a.src, tk) * a.src.row_stride_b;
+    const int p = position_of(a, tk);
+    const int64_t ut = (thetas(job) & 0xff) * a.theta_stride;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[t][i] = 0.f;
     for (int k = 0; k < S; ++k) {
-      __syncthreads();  // rows ready / previous member's reads done
-      const int pr = cload(a.pairs + static_cast<size_t>(job) * S + k);
-      gcptr sbase = layer_base(a.src, kind, pr & 0xffff) + static_cast<int64_t>((pr >> 16) - a.src.head_offset) * D * eb;
-      for (int e = threadIdx.x; e < kAnyTile * half; e += kAnyThreads) {
-        const int t = e / half, j = e % half;
-        const int pos = tpos[t];
-        const int64_t s = srow[t];
-        float x1 = 0.f, x2 = 0.f;
-        if (s >= 0) {
-          const CB_GLOBAL IO* row = reinterpret_cast<const CB_GLOBAL IO*>(sbase + s * a.src.row_stride_b);
-          x1 = AnyIO<IO>::get(row + j);
-          x2 = AnyIO<IO>::get(row + j + half);
+      const int pr = cload(a.pairs + static_cast<int64_t>(job) * S + k);
+      gcptr sb = layer_base(a.src, kind, pr & 0xffff) + static_cast<int64_t>((pr >> 16) - a.src.head_offset) * D * eb;
+      const CB_GLOBAL IO* row = reinterpret_cast<const CB_GLOBAL IO*>(sb + ro);
+      const CB_GLOBAL float* w = gtab(reinterpret_cast<const float*>(a.w)) +
+                                 static_cast<int64_t>(job) * NC * 2 * NG * kAnyFragU4 * 4;
+      for (int d = 0; d < D; ++d) {
+        const int j = d < half ? d : d - half;
+        const float x1 = AnyIO<IO>::get(row + j), x2 = AnyIO<IO>::get(row + j + half);
+        float x = d < half ? x1 : x2;
+        if (IS_K) {
+          const int64_t at = ut + static_cast<int64_t>(p) * HP + j;
+          const float c = gtab(a.ucos_tab)[at], s = gtab(a.usin_tab)[at];
+          x = d < half ? __builtin_fmaf(x1, c, x2 * s) : __builtin_fmaf(x2, c, -(x1 * s));
         }
-        if (is_k) {
-          const float c = ucos[static_cast<int64_t>(pos) * half + j];
-          const float sn = usin[static_cast<int64_t>(pos) * half + j];
-          const float k1 = __builtin_fmaf(x1, c, x2 * sn);
-          const float k2 = __builtin_fmaf(x2, c, -(x1 * sn));
-          x1 = k1;
-          x2 = k2;
-        }
-        xs[t][j] = x1;
-        xs[t][j + half] = x2;
-      }
-      __syncthreads();
-      if (active) {
-        const CB_GLOBAL float* wk_ = W + static_cast<int64_t>(k) * D * D;
-        for (int i = 0; i < D; ++i) {
-          const float w1 = wk_[static_cast<int64_t>(i) * D + p];
-          const float w2 = wk_[static_cast<int64_t>(i) * D + p + half];
 #pragma unroll
-          for (int m = 0; m < kAnyMaxTok; ++m) {
-            if (m < toks) {
-              const int t = sub + m * tpp;
-              if (t < kAnyTile) {
-                const float x = xs[t][i];
-                acc[m][0] = __builtin_fmaf(x, w1, acc[m][0]);
-                acc[m][1] = __builtin_fmaf(x, w2, acc[m][1]);
-              }
-            }
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            y[t][i] = __builtin_fmaf(x, w[any_w_offset(D, k, d, t * half + min(jo + i, half - 1))] *
+                                                (AnyIO<IO>::kScaled ? inv[t][i] : 1.f), y[t][i]);
+      }
+    }
+  };
+
+  // Bias, target RoPE (keys), cast and store of tile token t's outputs.
+  int64_t rtab = 0;      // rotation tables and target rows of the current tile
+  gptr tbase = nullptr;
+  auto rotation = [&](const AnyRows<TT>& r, int t, int jo, f32x4& c, f32x4& s) __attribute__((always_inline)) {
+    const int64_t at = rtab + static_cast<int64_t>(r.pos[t]) * HP + jo;
+    c = gload<f32x4>((gcptr)(gtab(a.cos_tab) + at));
+    s = gload<f32x4>((gcptr)(gtab(a.sin_tab) + at));
+  };
+  auto finish = [&](const AnyRows<TT>& r, char* stage, int t, int jo, const float (&bs)[2][4], const f32x4& c, const f32x4& s,
+                    float (&y)[2][4], bool keep) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[h][i] += bs[h][i];
+    if constexpr (IS_K) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float y1 = y[0][i], y2 = y[1][i];
+        y[0][i] = __builtin_fmaf(y1, c[i], -(y2 * s[i]));
+        y[1][i] = __builtin_fmaf(y2, c[i], y1 * s[i]);
+      }
+    }
+    if constexpr (STAGED) {
+      char* st = stage + t * kRowB + ((ng % NGW) * 16 + 4 * g) * 2;
+      if (keep)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          *reinterpret_cast<uint2*>(st + h * NGW * 32) =
+              make_uint2(AnyIO<IO>::pack(y[h][0], y[h][1]), AnyIO<IO>::pack(y[h][2], y[h][3]));
+      return;
+    }
+    const int64_t row = r.tgt[t];
+    if (row < 0 || jo >= half || !keep) return;
+    gptr out = tbase + row * a.tgt.row_stride_b + jo * eb;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      gptr o = out + h * half * eb;
+      if constexpr (WIDE && F32) {
+        gstore<f32x4>(o, f32x4{y[h][0], y[h][1], y[h][2], y[h][3]});
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (jo + i < half) gstore<IO>(o + i * eb, AnyIO<IO>::put(y[h][i]));
+      }
+    }
+  };
+
+  constexpr std::integral_constant<int, 0> part0{};
+  constexpr std::integral_constant<int, 1> part1{};
+  int buf = 0;
+  fetch_rows(cur);
+  load_w(cur.job, 0, part0);
+  load_w(cur.job, 0, part1);
+  more = advance(next);
+  finish_rows(cur, tab[0], true);
+  fetch_rows(next);
+  __syncthreads();
+  load_raw(tab[0]);
+  load_tab(tab[0], NC > 1 ? cur.job : next.job);
+  finish_rows(next, tab[1], more);
+  convert(xs);
+  int rb = 0;  // row table of the current tile
+  for (;;) {
+    then = next;
+    more2 = more && advance(then);
+    fetch_rows(then);
+    // Column tiles of this wave that hold tokens (none past the last group).
+    const int left = cur.hi - cur.lo - mg * 16 * CT;
+    const int nct = busy ? min(CT, max(0, (left + 15) >> 4)) : 0;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        acc[t][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (F32) acc_b[t][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    for (int c = 0; c < NC; ++c) {
+      const bool last = c + 1 == NC;
+      const int cn = last ? 0 : c + 1;
+      const int jn = last ? next.job : cur.job;  // job of the chunk to gather
+      __syncthreads();  // this chunk is in its buffer, the one before it has been read
+      // The loads are unconditional (without a next tile, `next` repeats this
+      // one): a branch around them would make the compiler wait for them where
+      // its paths join.
+      const AnyRows<TT>& r = tab[last && more ? (rb + 1) % kAnyRowBufs : rb];
+      // (Element-wise loads have no registers to wait in: they come last.)
+      const int jt = c + 2 < NC ? cur.job : last && NC == 1 ? then.job : next.job;
+      const uint4* xb = xs + buf * kBuf;
+      if constexpr (WIDE) load_raw(r);
+      multiply(xb, part0, nct);
+      load_w(jn, cn, part0);
+      if constexpr (WIDE) load_tab(r, jt);
+      multiply(xb, part1, nct);
+      load_w(jn, cn, part1);
+      if constexpr (!WIDE) {
+        load_raw(r);
+        load_tab(r, jt);
+      }
+      if (last) finish_rows(then, tab[(rb + 2) % kAnyRowBufs], more2);
+      buf ^= 1;
+      convert(xs + buf * kBuf);
+    }
+    // Epilogue: scale, then bias, target RoPE (keys), cast, store.
+    char* stage = reinterpret_cast<char*>(xs + (buf ^ 1) * kBuf);
+    const int jo = hide(jo_);
+    {
+      const int mx = cload(reinterpret_cast<const int*>(a.jobs + cur.job));
+      tbase = const_cast<gptr>(layer_base(a.tgt, kind, mx & 0xffff)) +
+              static_cast<int64_t>((mx >> 16) - a.tgt.head_offset) * D * eb;
+      rtab = (thetas(cur.job) >> 8 & 0xff) * a.theta_stride;
+    }
+    float inv[2][4], bs[2][4];
+    if constexpr (AnyIO<IO>::kScaled) out_values(a.wscale, cur.job, jo, inv);
+    out_values(a.bias, cur.job, jo, bs);
+    __syncthreads();  // the tile's last chunk has been read: its buffer takes the outputs
+    uint32_t again = 0;  // column tiles whose outputs are not finite
+    constexpr int GC = CT < 4 ? CT : 4;  // column tiles whose rotation values are requested together
+#pragma unroll
+    for (int c0 = 0; c0 < CT; c0 += GC) {
+      if (c0 >= nct) continue;
+      f32x4 rc[GC], rs[GC];
+      if constexpr (IS_K) {
+#pragma unroll
+        for (int cc = 0; cc < GC; ++cc) rotation(tab[rb], mg * 16 * CT + 16 * (c0 + cc) + col, jo, rc[cc], rs[cc]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int cc = 0; cc < GC; ++cc) {
+        const int ct = c0 + cc;
+        if (ct >= nct) continue;
+        float y[2][4];
+        float fin = 0.f;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            y[h][i] = acc[h][ct][i];
+            if constexpr (F32) y[h][i] += acc_b[h][ct][i];
+            if constexpr (AnyIO<IO>::kScaled) y[h][i] *= inv[h][i] * (IS_K ? 1.f / AnyIO<IO>::kKeyScale : 1.f);
+            fin = __builtin_fmaf(y[h][i], 0.f, fin);
           }
-        }
+        const bool bad = !F32 && fin != 0.f;
+        if (bad) again |= 1u << ct;
+        finish(tab[rb], stage, mg * 16 * CT + 16 * ct + col, jo, bs, rc[cc], rs[cc], y, !bad);
       }
     }
-    if (active) {
-      const float b1 = bias[p], b2 = bias[p + half];
-#pragma unroll
-      for (int m = 0; m < kAnyMaxTok; ++m) {
-        if (m >= toks) continue;
-        const int t = sub + m * tpp;
-        if (t >= n) continue;
-        const int64_t row = trow[t];
-        if (row < 0) continue;
-        float y1 = acc[m][0] + b1, y2 = acc[m][1] + b2;
-        if (is_k) {
-          const int pos = tpos[t];
-          const float c = rcos[static_cast<int64_t>(pos) * half + p];
-          const float sn = rsin[static_cast<int64_t>(pos) * half + p];
-          const float r1 = __builtin_fmaf(y1, c, -(y2 * sn));
-          const float r2 = __builtin_fmaf(y2, c, y1 * sn);
-          y1 = r1;
-          y2 = r2;
-        }
-        CB_GLOBAL IO* out = reinterpret_cast<CB_GLOBAL IO*>(tbase + row * a.tgt.row_stride_b);
-        AnyIO<IO>::put(out + p, y1);
-        AnyIO<IO>::put(out + p + half, y2);
+    if (!F32 && __builtin_amdgcn_ballot_w64(again != 0)) {
+      for (int ct = 0; ct < nct; ++ct) {
+        if (!(again >> ct & 1)) continue;
+        const int t = mg * 16 * CT + 16 * ct + col;
+        if (tab[rb].tgt[t] < 0) continue;
+        float y[2][4];
+        const int js = hide(jo_);
+        slow(cur.lo + t, js, inv, y);
+        f32x4 c = {}, sn = {};
+        if constexpr (IS_K) rotation(tab[rb], t, js, c, sn);
+        finish(tab[rb], stage, t, js, bs, c, sn, y, true);
       }
     }
+    if constexpr (STAGED) {
+      // Whole rows to the pool: a token's dims of one half are NGW * 2 pieces
+      // of 16 bytes, consecutive lanes storing consecutive pieces.
+      constexpr int PPR = NGW * 4;
+      __syncthreads();
+#pragma unroll 4
+      for (int i = threadIdx.x; i < TT * PPR; i += NW * kWave) {
+        const int t = i / PPR, pc = i % PPR, h = pc / (NGW * 2);
+        const int j = static_cast<int>(blockIdx.y) * NGW * 16 + (pc % (NGW * 2)) * 8;
+        const int64_t row = tab[rb].tgt[t];
+        if (row >= 0 && j < half && t < cur.hi - cur.lo)
+          gstore<uint4>(tbase + row * a.tgt.row_stride_b + (h * half + j) * eb,
+                        *reinterpret_cast<const uint4*>(stage + t * kRowB + pc * 16));
+      }
+    }
+    if (!more) break;
+    rb = (rb + 1) % kAnyRowBufs;
+    cur = next;
+    next = then;
+    more = more2;
   }
   if (errbits) atomicOr(a.err, errbits);
 }
 
-// Plan data of the generic kernel: W [job][s*D][D] and bias [job][D] copied
-// in sorted job order.
-__global__ void copy_weights_kernel(const float* __restrict__ w, const float* __restrict__ bias,
-                                    const int32_t* __restrict__ order, int njobs, int per_job_w, int D,
-                                    float* __restrict__ wp, float* __restrict__ bp) {
-  const int64_t total = static_cast<int64_t>(njobs) * per_job_w;
-  for (int64_t idx = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; idx < total;
-       idx += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const int64_t j = idx / per_job_w;
-    wp[idx] = w[static_cast<int64_t>(order[j]) * per_job_w + idx % per_job_w];
+// NW waves; a wave covers CT column tiles of its 16 output pairs. One
+// workgroup per CU of 8 waves, two of 4.
+template <typename IO, int NW, int CT>
+__global__ __launch_bounds__(NW * kWave, 2) void map_install_any_kernel(MapArgs a, int D) {
+  __shared__ uint4 xs[2 * any_buf_u4(NW, NW * 16 * CT / any_tokens(NW), AnyIO<IO>::kTerms, sizeof(IO) == 4)];
+  __shared__ AnyRows<any_tokens(NW)> tab[kAnyRowBufs];
+  const int x = blockIdx.x & 7, nwg = gridDim.x >> 3;
+  int p = blockIdx.x >> 3;
+  const bool wide = any_wide(a, D);
+  AnySegment sg;
+  for (int seg = 0; any_segment(a, x, seg, &sg); ++seg) {
+    if (p < sg.count) {
+      if (wide && !(seg & 1)) any_run<IO, NW, CT, true, true>(a, D, sg, p, nwg, xs, tab);
+      else if (wide) any_run<IO, NW, CT, false, true>(a, D, sg, p, nwg, xs, tab);
+      else if (!(seg & 1)) any_run<IO, NW, CT, true, false>(a, D, sg, p, nwg, xs, tab);
+      else any_run<IO, NW, CT, false, false>(a, D, sg, p, nwg, xs, tab);
+      p += (sg.count - p + nwg - 1) / nwg * nwg;
+      __syncthreads();  // the row tables and buffers are free again
+    }
+    p -= sg.count;
   }
-  const int64_t nb = static_cast<int64_t>(njobs) * D;
-  for (int64_t idx = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; idx < nb;
-       idx += static_cast<int64_t>(gridDim.x) * blockDim.x)
-    bp[idx] = bias[static_cast<int64_t>(order[idx / D]) * D + idx % D];
+}
+
+// Plan data of the general kernel: W in fragment order (any_w_offset, padded
+// entries zero), for fp16 with every output dim scaled by the power of two
+// that brings its largest weight into [2^13, 2^14), the inverse scales, and
+// the bias, in sorted job order. One workgroup per job.
+__global__ __launch_bounds__(256) void pack_any_kernel(const float* __restrict__ w, const float* __restrict__ bias,
+                                                       const int32_t* __restrict__ order, int S, int D, int scaled,
+                                                       float* __restrict__ wp, float* __restrict__ bp,
+                                                       float* __restrict__ sp) {
+  __shared__ float scale[kAnyMaxDim];
+  const int64_t job = blockIdx.x, from = order[job];
+  const float* src = w + from * S * D * D;
+  for (int o = threadIdx.x; o < D; o += blockDim.x) {
+    float sc = 1.f;
+    if (scaled) {
+      float m = 0.f;
+      for (int i = 0; i < S * D; ++i) m = fmaxf(m, fabsf(src[static_cast<int64_t>(i) * D + o]));
+      int e = 0;
+      if (m > 0.f && m < INFINITY) {
+        (void)frexpf(m, &e);  // m in [2^(e-1), 2^e)
+        sc = ldexpf(1.f, min(max(14 - e, -100), 100));
+      }
+    }
+    scale[o] = sc;
+    sp[job * D + o] = 1.f / sc;
+    bp[job * D + o] = bias[from * D + o];
+  }
+  __syncthreads();
+  const int Q = any_chunks(D), NG = any_groups(D), half = D / 2;
+  const int64_t total = static_cast<int64_t>(S) * Q * 2 * NG * kAnyFragU4 * 4;
+  float* dst = wp + job * total;
+  for (int64_t idx = threadIdx.x; idx < total; idx += blockDim.x) {
+    int64_t rem = idx;
+    const int e0 = rem % 4; rem /= 4;
+    const int lane = rem % kWave; rem /= kWave;
+    const int e = e0 + 4 * static_cast<int>(rem % 2); rem /= 2;
+    const int tile = rem % 2; rem /= 2;
+    const int ng = rem % NG; rem /= NG;
+    const int part = rem % 2; rem /= 2;
+    const int q = rem % Q; rem /= Q;
+    const int k = static_cast<int>(rem);
+    const int jp = 32 * q + 8 * (lane >> 4) + e, op = 16 * ng + (lane & 15);
+    const int i = k * D + part * half + jp, o = tile * half + op;
+    dst[idx] = jp < half && op < half ? src[static_cast<int64_t>(i) * D + o] * scale[o] : 0.f;
+  }
 }
 
 // Plan tables from standard [theta][pos][D/2] cos/sin: rotation tables and
 // un-rotation tables cos/m, sin/m (m = max(cos^2 + sin^2, FLT_MIN)), both in
 // the permuted half-row layout; also max |m - 1| per theta set (as float bits).
+// natural > 0: row-major with rows of `natural` values instead (general kernel).
 // Grid: (blocks per theta set, theta sets); each block reduces its maximum in
 // LDS and issues one atomic.
 __global__ __launch_bounds__(256) void prepare_tables_kernel(
@@ -1988,7 +2578,7 @@ __global__ __launch_bounds__(256) void prepare_tables_kernel(
     const float cc = c[i], ss = s[i];
     const float m = fmaxf(cc * cc + ss * ss, 1.17549435e-38f);
     const int64_t o = blockIdx.y * out_per_theta +
-                      (natural ? k : tab_offset(half, k / half, static_cast<int>(k % half)));
+                      (natural ? k / half * natural + k % half : tab_offset(half, k / half, static_cast<int>(k % half)));
     rc[o] = cc;
     rs[o] = ss;
     uc[o] = cc / m;
@@ -2332,10 +2922,12 @@ struct cb_plan {
   int window_size[kMaxClasses] = {0, 0, 0, 0};
   int cls_unit_begin[kMaxClasses] = {0, 0, 0, 0};
   int cls_unit_end[kMaxClasses] = {0, 0, 0, 0};
+  int cls_val_begin[kMaxClasses] = {0, 0, 0, 0};  // general kernel: first values unit
   int max_src_layer = 0, min_src_head = 0, max_src_head = 0;
   int max_tgt_layer = 0, min_tgt_head = 0, max_tgt_head = 0;
   void* d_w = nullptr;
   float* d_bias = nullptr;
+  float* d_scale = nullptr;  // general kernel: inverse weight scales
   int4* d_jobs = nullptr;
   int32_t* d_pairs = nullptr;
   int32_t* d_unit_job = nullptr;
@@ -2383,7 +2975,7 @@ namespace {
 
 void plan_free(cb_plan* p) {
   if (!p) return;
-  void* ptrs[] = {p->d_w,         p->d_bias,         p->d_jobs,           p->d_pairs,
+  void* ptrs[] = {p->d_w,         p->d_bias,         p->d_scale,          p->d_jobs,           p->d_pairs,
                   p->d_unit_job,  p->d_unit_njobs,   p->d_unit_group,     p->d_group_unit_start,
                   p->d_group_unit_count, p->d_cos,   p->d_sin,            p->d_ucos,
                   p->d_usin,      p->d_err,          p->d_sink,
@@ -2418,7 +3010,7 @@ int to_dev_rows(const cb_rows& r, int elem_bytes, DevRows* out, int align = 16) 
   out->index_kind = r.index_kind;
   out->page_size = r.page_size;
   out->head_offset = r.head_offset;
-  out->pad = 0;
+  out->layers = r.num_layers;
   if (r.index_kind < CB_INDEX_IDENTITY || r.index_kind > CB_INDEX_BLOCK_TABLE)
     return fail(CB_EINVAL, "unknown index_kind %d", r.index_kind);
   if (r.index_kind != CB_INDEX_IDENTITY && !r.index)
@@ -2509,6 +3101,11 @@ int plan_build(const cb_plan_desc* d, const std::vector<int>& order, const std::
   for (int c = 0; c < d->num_windows; ++c)
     if (p->cls_unit_begin[c] < 0) p->cls_unit_begin[c] = p->cls_unit_end[c] = 0;
   p->num_units = static_cast<int>(unit_job.size());
+  for (int c = 0; c < d->num_windows; ++c) {
+    int u = p->cls_unit_begin[c];
+    while (u < p->cls_unit_end[c] && (jobs[unit_job[u]].y & 0xff) == CB_KIND_K) ++u;
+    p->cls_val_begin[c] = u;
+  }
   if (p->support_gemm) {
     // The support kernel gives XCD x units x, x + 8, ... of each class. Place
     // the units so that these are a contiguous run of the sorted keys jobs
@@ -2549,10 +3146,13 @@ int plan_build(const cb_plan_desc* d, const std::vector<int>& order, const std::
     p->num_cus = std::max(8, std::min(cus, kMaxStreamBlocks) / 8 * 8);
   }
 
-  const size_t w_bytes = p->generic ? static_cast<size_t>(nj) * S * D * D * 4
+  const size_t w_bytes = p->generic ? static_cast<size_t>(nj) * S * any_chunks(D) * 2 * any_groups(D) * kAnyFragU4 * 16
                                     : static_cast<size_t>(nj) * S * (D / 16) * (D / 32) * p->ntw * kWave * 8 * 2;
   const int64_t padded_positions = (static_cast<int64_t>(d->table_positions) + kTabBlock - 1) / kTabBlock * kTabBlock;
-  const size_t table = static_cast<size_t>(d->num_thetas) * padded_positions * (D / 2);
+  // Values per position of the plan's tables: the general kernel pads its
+  // rows with zeros to whole 32-pair chunks.
+  const int table_row = p->generic ? 32 * any_chunks(D) : D / 2;
+  const size_t table = static_cast<size_t>(d->num_thetas) * padded_positions * table_row;
   int rc;
   if ((rc = upload(&p->d_pairs, pairs.data(), pairs.size() * 4, &bytes))) return rc;
   if ((rc = upload(&p->d_unit_job, unit_job.data(), unit_job.size() * 4, &bytes))) return rc;
@@ -2568,6 +3168,9 @@ int plan_build(const cb_plan_desc* d, const std::vector<int>& order, const std::
   if ((rc = upload(&p->d_usin, nullptr, table * 4, &bytes))) return rc;
   if ((rc = upload(&p->d_err, nullptr, 4, &bytes))) return rc;
   if ((rc = upload(&p->d_sink, nullptr, kSinkBytes + kZeroBytes, &bytes))) return rc;
+  if (p->generic && (rc = upload(&p->d_scale, nullptr, static_cast<size_t>(nj) * D * 4, &bytes))) return rc;
+  if (table_row != D / 2)
+    for (float* t : {p->d_cos, p->d_sin, p->d_ucos, p->d_usin}) CB_HIP(hipMemset(t, 0, table * 4));
   CB_HIP(hipMemset(p->d_err, 0, 4));
   CB_HIP(hipMemset(static_cast<char*>(p->d_sink) + kSinkBytes, 0, kZeroBytes));
   // Rotation / un-rotation tables in the permuted layout, and which theta sets
@@ -2580,8 +3183,8 @@ int plan_build(const cb_plan_desc* d, const std::vector<int>& order, const std::
     if (e == hipSuccess) {
       hipLaunchKernelGGL(prepare_tables_kernel, dim3(256, d->num_thetas), dim3(256), 0, 0,
                          d->d_cos, d->d_sin, p->d_cos, p->d_sin, p->d_ucos, p->d_usin, D / 2,
-                         static_cast<int64_t>(d->table_positions) * (D / 2), padded_positions * (D / 2), d_norm,
-                         p->generic ? 1 : 0);
+                         static_cast<int64_t>(d->table_positions) * (D / 2), padded_positions * table_row, d_norm,
+                         p->generic ? table_row : 0);
       e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpy(norm.data(), d_norm, norm.size() * sizeof(unsigned), hipMemcpyDeviceToHost);
@@ -2626,8 +3229,8 @@ int plan_build(const cb_plan_desc* d, const std::vector<int>& order, const std::
   if (e == hipSuccess) {
     uint16_t* wp = static_cast<uint16_t*>(p->d_w);
     if (p->generic)
-      hipLaunchKernelGGL(copy_weights_kernel, dim3(1024), dim3(256), 0, 0, d->d_weight, d->d_bias, d_order,
-                         nj, S * D * D, D, static_cast<float*>(p->d_w), p->d_bias);
+      hipLaunchKernelGGL(pack_any_kernel, dim3(nj), dim3(256), 0, 0, d->d_weight, d->d_bias, d_order, S, D,
+                         d->io_dtype == CB_DTYPE_F16 ? 1 : 0, static_cast<float*>(p->d_w), p->d_bias, p->d_scale);
     else if (D == 64 && p->ntw == 2)
       launch_pack<64, 2>(d, d_order, wp, p->d_bias);
     else if (D == 64)
@@ -2656,10 +3259,22 @@ int plan_build(const cb_plan_desc* d, const std::vector<int>& order, const std::
   return CB_OK;
 }
 
+// General kernel: waves per workgroup, column tiles per wave and workgroups
+// that share a job's output groups.
+struct AnyShape {
+  int waves, tiles, blocks;
+};
+AnyShape any_shape(int D, bool f32) {
+  const int ng = any_groups(D);
+  if (ng > 4 && !f32) return {8, 8, (ng + 7) / 8};
+  if (ng > 2) return {4, 4, (ng + 3) / 4};
+  return {4, 2, 1};
+}
+
 // Default tokens per workgroup: about three workgroups per CU over the launch
 // (one resident per CU for the streaming kernel), at least 512 tokens.
 int default_chunk(const cb_plan* p, int n) {
-  if (p->generic) return 8 * kAnyTile;
+  if (p->generic) return any_tokens(any_shape(p->info.head_dim, p->elem_bytes == 4).waves);
   if (p->info.support != 1) return kGenSubTokens;
   int64_t units = 0;
   for (int c = 0; c < p->num_windows; ++c) units += p->cls_unit_end[c] - p->cls_unit_begin[c];
@@ -2858,6 +3473,20 @@ void split_cost_line(const cb_plan* p, MapArgs* a, bool allow_pool) {
   a->pool_gs = static_cast<int32_t>(gs);
 }
 
+template <typename IO>
+void launch_any(int D, int64_t items, hipStream_t s, const MapArgs& a) {
+  const AnyShape sh = any_shape(D, sizeof(IO) == 4);
+  const dim3 g(static_cast<unsigned>(items), static_cast<unsigned>(sh.blocks)), b(sh.waves * kWave);
+  if constexpr (sizeof(IO) == 2) {
+    if (sh.waves == 8) {
+      hipLaunchKernelGGL((map_install_any_kernel<IO, 8, 8>), g, b, 0, s, a, D);
+      return;
+    }
+  }
+  if (sh.tiles == 4) hipLaunchKernelGGL((map_install_any_kernel<IO, 4, 4>), g, b, 0, s, a, D);
+  else hipLaunchKernelGGL((map_install_any_kernel<IO, 4, 2>), g, b, 0, s, a, D);
+}
+
 // Enqueue the map kernel over class token ranges [first[c], first[c] +
 // count[c]) of the launch's token space. `a` carries the two sides (and, for
 // batches, the position vector); the plan fields are filled in here.
@@ -2872,8 +3501,10 @@ int launch_map(const cb_plan* p, MapArgs& a, const int64_t* first, const int64_t
     return fail(CB_EINVAL, "tokens_per_workgroup must be a positive multiple of %d", unit);
   // The support kernel's items are fixed 256-token blocks; the knob does not apply.
   if (p->support_gemm) chunk = kSupTile;
+  if (p->generic) chunk = std::min(chunk, any_tokens(any_shape(D, p->elem_bytes == 4).waves));
   a.w = static_cast<const uint4*>(p->d_w);
   a.bias = p->d_bias;
+  a.wscale = p->d_scale;
   a.jobs = p->d_jobs;
   a.pairs = p->d_pairs;
   a.unit_job = p->d_unit_job;
@@ -2885,7 +3516,8 @@ int launch_map(const cb_plan* p, MapArgs& a, const int64_t* first, const int64_t
   a.sin_tab = p->d_sin;
   a.ucos_tab = p->d_ucos;
   a.usin_tab = p->d_usin;
-  a.theta_stride = (static_cast<int64_t>(p->info.table_positions) + kTabBlock - 1) / kTabBlock * kTabBlock * (D / 2);
+  a.theta_stride = (static_cast<int64_t>(p->info.table_positions) + kTabBlock - 1) / kTabBlock * kTabBlock *
+                   (p->generic ? 32 * any_chunks(D) : D / 2);
   a.support = p->info.support;
   a.chunk = chunk;
   a.err = p->d_err;
@@ -2898,6 +3530,7 @@ int launch_map(const cb_plan* p, MapArgs& a, const int64_t* first, const int64_t
     const int64_t nch = (count[c] + chunk - 1) / chunk;
     a.cls_unit_begin[c] = p->cls_unit_begin[c];
     a.cls_unit_end[c] = p->cls_unit_end[c];
+    a.cls_val_begin[c] = p->cls_val_begin[c];
     a.cls_tok_first[c] = static_cast<int32_t>(first[c]);
     a.cls_tok_count[c] = static_cast<int32_t>(count[c]);
     a.cls_nchunks[c] = static_cast<int32_t>(std::max<int64_t>(nch, 1));
@@ -2912,6 +3545,8 @@ int launch_map(const cb_plan* p, MapArgs& a, const int64_t* first, const int64_t
   a.total_items = static_cast<int32_t>(items);
   a.padded_items = static_cast<int32_t>((items + 7) / 8 * 8);
   int64_t grid_blocks = a.padded_items;
+  if (p->generic)  // persistent: one workgroup of 8 waves per CU, or two of 4
+    grid_blocks = std::min<int64_t>(grid_blocks, static_cast<int64_t>(p->num_cus) * (8 / any_shape(D, p->elem_bytes == 4).waves));
   // Held from the cost-line split through the launch and its pair event.
   std::unique_lock<std::mutex> held;
   int tracked_pair = -1;
@@ -3002,10 +3637,9 @@ int launch_map(const cb_plan* p, MapArgs& a, const int64_t* first, const int64_t
       p->pair_stream[tracked_pair] = s;
     }
   } else if (p->generic) {
-    const dim3 g(static_cast<unsigned>(grid_blocks)), b(kAnyThreads);
-    if (p->info.io_dtype == CB_DTYPE_BF16) hipLaunchKernelGGL(map_install_any_kernel<uint16_t>, g, b, 0, s, a, D);
-    else if (p->info.io_dtype == CB_DTYPE_F16) hipLaunchKernelGGL(map_install_any_kernel<_Float16>, g, b, 0, s, a, D);
-    else hipLaunchKernelGGL(map_install_any_kernel<float>, g, b, 0, s, a, D);
+    if (p->info.io_dtype == CB_DTYPE_BF16) launch_any<uint16_t>(D, grid_blocks, s, a);
+    else if (p->info.io_dtype == CB_DTYPE_F16) launch_any<_Float16>(D, grid_blocks, s, a);
+    else launch_any<float>(D, grid_blocks, s, a);
   } else if (p->support_gemm) {
     // One persistent workgroup per CU; 8 per XCD at least.
     const unsigned per_xcd = static_cast<unsigned>(std::max(1, p->num_cus / 8));

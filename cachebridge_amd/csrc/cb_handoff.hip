@@ -346,6 +346,7 @@ struct MapArgs {
   int32_t ncls;
   int32_t cls_unit_begin[kMaxClasses];
   int32_t cls_val_begin[kMaxClasses];  // general kernel: first values unit of each class
+  int32_t cls_job_begin[kMaxClasses];  // short kernel: first job of each class
   int32_t cls_tok_first[kMaxClasses];
   int32_t cls_tok_count[kMaxClasses];
   int32_t cls_nchunks[kMaxClasses];
@@ -1020,6 +1021,222 @@ __global__ __launch_bounds__(kStreamThreads) void map_install_stream_kernel(MapA
       atomicOr(a.err, 8);
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// Short-request kernel (support 1, the streaming kernel's shapes and packing).
+//
+// A request of up to a few hundred tokens is bound by reading the maps once
+// and by the latency of a workgroup's start, not by its products: the
+// streaming kernel's chain of index words, W into LDS, barrier and first
+// products takes 11 us at any length, and its two-job units leave CUs idle or
+// stage one W on several of them. Here a workgroup of four waves takes one job
+// and a chunk of the tokens. A wave owns one pair of row tiles (16 output dims
+// of each half that hold RoPE partners) and requests its part of the job's W
+// straight into registers before anything else. The tokens pass in rounds of
+// 64: each wave gathers, un-rotates and splits one 16-token sub-tile into LDS
+// in fragment order (two buffers, one barrier a round), then multiplies the
+// round's sub-tiles. At D 64 a job has two pairs, each shared by two
+// waves that take half of the round's sub-tiles.
+//
+// Products, bias and rotations are the streaming kernel's, in its order, so a
+// job's rows are bit-identical whichever of the two maps them.
+// ---------------------------------------------------------------------------
+
+constexpr int kRoundTokens = kWaves * kSubTokens;
+
+template <int D, typename IO>
+struct ShortLds {
+  static constexpr int XT = IOTraits<IO>::XT_K;
+  uint4 x[2][kWaves][Gm<D, IO>::KS][XT][kWave];  // split sub-tiles of two rounds
+  int32_t row[2][kRoundTokens];                  // target rows (-1: nothing is written)
+  int32_t pos[2][kRoundTokens];
+};
+
+template <int D, typename IO, bool IS_K>
+__device__ __attribute__((always_inline)) inline void short_run(const MapArgs& a, ShortLds<D, IO>& L, int job, int lo, int hi) {
+#pragma clang fp contract(off)
+  using C = Gm<D, IO>;
+  using T = IOTraits<IO>;
+  constexpr int NTW = C::NTW, XT = IS_K ? T::XT_K : T::XT_V;
+  constexpr int KS = C::KS, RT = C::RT, G = C::G, HALF = C::HALF;
+  constexpr int kind = IS_K ? CB_KIND_K : CB_KIND_V;
+  constexpr int TG = IS_K ? G : 1;
+  constexpr int PAIRS = D / 32;              // row-tile pairs of a job
+  constexpr int SPLIT = kWaves / PAIRS;      // waves per pair
+  constexpr int NS = kWaves / SPLIT;         // sub-tiles of a round a wave multiplies
+  const int lane = threadIdx.x & (kWave - 1), g = lane >> 4, col = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int pair = wave % PAIRS, s0 = wave / PAIRS * NS;
+  const int* jm = reinterpret_cast<const int*>(a.jobs + job);
+  const int mx = cload(jm), meta_y = cload(jm + 1), meta_z = cload(jm + 2), pr = cload(a.pairs + job);
+  const CB_GLOBAL uint32_t* spare = reinterpret_cast<const CB_GLOBAL uint32_t*>(as_global(a.sink));
+
+  // Index words of this wave's sub-tile of the round at t0 (tokens past the
+  // end repeat the last).
+  uint2 fs, fd;
+  int32_t fp;
+  auto token = [&](int t0) __attribute__((always_inline)) { return t0 + wave * kSubTokens + col; };
+  auto fetch_rows = [&](int t0) __attribute__((always_inline)) {
+    const int t = min(token(t0), hi - 1);
+    fs = row_fetch(a.src, t, spare);
+    fd = row_fetch(a.tgt, t, spare);
+    fp = static_cast<int32_t>(*(a.pos ? reinterpret_cast<const CB_GLOBAL uint32_t*>(as_global(a.pos)) + t : spare));
+  };
+  fetch_rows(lo);
+  // W fragments of row tiles `pair` and its partner, and their bias.
+  bf16x8 wf[2][KS][NTW];
+  f32x4 bq[2];
+  {
+    gcptr w = as_global(a.w + static_cast<size_t>(job) * C::W_U4) + lane * 16;
+    const CB_GLOBAL float* b = gtab(a.bias) + static_cast<int64_t>(job) * D + gen_out_dim(D, pair, 4 * g);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int p = 0; p < NTW; ++p)
+          wf[t][ks][p] = __builtin_bit_cast(
+              bf16x8, gload<uint4>(w + ((pair + t * (RT / 2)) * KS * NTW + ks * NTW + p) * (kWave * 16)));
+#pragma unroll
+    for (int t = 0; t < 2; ++t) bq[t] = gload<f32x4>((gcptr)(b + t * HALF));
+  }
+  gcptr sbase = layer_base(a.src, kind, pr & 0xffff) + static_cast<int64_t>((pr >> 16) - a.src.head_offset) * D * C::BYTES;
+  gptr tbase = const_cast<gptr>(layer_base(a.tgt, kind, mx & 0xffff)) +
+               static_cast<int64_t>((mx >> 16) - a.tgt.head_offset) * D * C::BYTES + gen_out_dim(D, pair, 4 * g) * C::BYTES;
+  const int64_t sth = ((meta_y >> 16) & 0xff) * a.theta_stride, tth = ((meta_y >> 24) & 0xff) * a.theta_stride;
+  const bool shared = (meta_z & kJobSharedTables) != 0;
+  const CB_GLOBAL float* ucos = gtab(shared ? a.cos_tab : a.ucos_tab) + sth;
+  const CB_GLOBAL float* usin = gtab(shared ? a.sin_tab : a.usin_tab) + sth;
+  const CB_GLOBAL float* rcos = gtab(a.cos_tab) + tth;
+  const CB_GLOBAL float* rsin = gtab(a.sin_tab) + tth;
+
+  int errbits = 0;
+  int32_t trow, tpos;  // of this lane's token in the round requested last
+  uint4 xr[2][C::RUN_U4];
+  float uc[TG], us[TG];
+  // Resolve the fetched rows of the round at t0 and request its inputs.
+  auto request = [&](int t0) __attribute__((always_inline)) {
+    const int t = min(token(t0), hi - 1);
+    const bool live = token(t0) < hi;
+    const int64_t s = row_finish(a.src, t, fs), d = row_finish(a.tgt, t, fd);
+    const bool sok = s >= 0 && s < a.src.rows, dok = d >= 0 && d < a.tgt.rows;
+    errbits |= live ? (sok ? 0 : 1) | (dok ? 0 : 2) : 0;
+    // A token whose source row is out of range writes nothing.
+    trow = live && sok && dok ? static_cast<int32_t>(d) : -1;
+    tpos = a.pos ? fp : a.position_start + t;
+    gcptr p = (live && sok ? sbase + s * a.src.row_stride_b : as_global(a.zero)) + g * G * C::BYTES;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int u = 0; u < C::RUN_U4; ++u) xr[h][u] = gload<uint4>(p + (h * HALF + u * C::E16) * C::BYTES);
+    if constexpr (IS_K) {
+      load_tab<G>(ucos, tpos, g, uc);
+      load_tab<G>(usin, tpos, g, us);
+    }
+  };
+  request(lo);
+  fetch_rows(lo + kRoundTokens);
+  int buf = 0;
+  for (int t0 = lo; t0 < hi; t0 += kRoundTokens, buf ^= 1) {
+    auto put = [&](int ks, int x, const uint4& v) __attribute__((always_inline)) { L.x[buf][wave][ks][x][lane] = v; };
+    if constexpr (!IS_K && XT == 1 && C::BYTES == 2) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) put(ks, 0, xr[ks / (KS / 2)][ks % (KS / 2)]);
+    } else {
+      float x1[G], x2[G];
+#pragma unroll
+      for (int u = 0; u < C::RUN_U4; ++u) {
+        unpack16<IO>(xr[0][u], x1 + u * C::E16);
+        unpack16<IO>(xr[1][u], x2 + u * C::E16);
+      }
+      if constexpr (IS_K) {
+#pragma unroll
+        for (int e = 0; e < G; ++e) {
+          const float k1 = __builtin_fmaf(x1[e], uc[e], x2[e] * us[e]);
+          const float k2 = __builtin_fmaf(x2[e], uc[e], -(x1[e] * us[e]));
+          x1[e] = k1;
+          x2[e] = k2;
+        }
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        uint32_t tw[XT][4];
+        split_terms<XT, 8>((ks / (KS / 2) ? x2 : x1) + (ks % (KS / 2)) * 8, tw);
+#pragma unroll
+        for (int x = 0; x < XT; ++x) put(ks, x, make_uint4(tw[x][0], tw[x][1], tw[x][2], tw[x][3]));
+      }
+    }
+    if (lane < kSubTokens) {
+      L.row[buf][wave * kSubTokens + lane] = trow;
+      L.pos[buf][wave * kSubTokens + lane] = tpos;
+    }
+    __syncthreads();  // the round is in LDS (and every wave is done with the round before the last)
+    f32x4 rc[NS], rs[NS];
+    if constexpr (IS_K) {
+#pragma unroll
+      for (int i = 0; i < NS; ++i) {
+        const int64_t off = tab_chunk<G>(L.pos[buf][(s0 + i) * kSubTokens + col], pair, g);
+        rc[i] = gload<f32x4>((gcptr)(rcos + off));
+        rs[i] = gload<f32x4>((gcptr)(rsin + off));
+      }
+    }
+    // The next round's inputs (past the end: the last token's again).
+    request(t0 + kRoundTokens);
+    fetch_rows(t0 + 2 * kRoundTokens);
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      const int st = s0 + i;
+      if (t0 + st * kSubTokens >= hi) break;
+      f32x4 acc[2];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        bf16x8 bx[XT];
+#pragma unroll
+        for (int x = 0; x < XT; ++x) bx[x] = __builtin_bit_cast(bf16x8, L.x[buf][st][ks][x][lane]);
+        int pi = 0;
+        for_products<XT, NTW>([&](int ii, int jj) {
+#pragma unroll
+          for (int t = 0; t < 2; ++t) acc[t] = mfma(wf[t][ks][jj], bx[ii], ks == 0 && pi == 0 ? bq[t] : acc[t]);
+          ++pi;
+        });
+      }
+      float o1[4] = {acc[0][0], acc[0][1], acc[0][2], acc[0][3]}, o2[4] = {acc[1][0], acc[1][1], acc[1][2], acc[1][3]};
+      if constexpr (IS_K) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float y1 = o1[e], y2 = o2[e];
+          o1[e] = __builtin_fmaf(y1, rc[i][e], -(y2 * rs[i][e]));
+          o2[e] = __builtin_fmaf(y2, rc[i][e], y1 * rs[i][e]);
+        }
+      }
+      const int32_t row = L.row[buf][st * kSubTokens + col];
+      if (row >= 0) {
+        gptr p = tbase + static_cast<int64_t>(row) * a.tgt.row_stride_b;
+        store_elems<IO, 4>(p, o1);
+        store_elems<IO, 4>(p + HALF * C::BYTES, o2);
+      }
+    }
+  }
+  if (errbits) atomicOr(a.err, errbits);
+}
+
+template <int D, typename IO>
+__global__ __launch_bounds__(kThreads, 2) void map_install_short_kernel(MapArgs a) {
+  // Items, class by class: job, token chunk. XCD x runs a contiguous eighth,
+  // so the chunks of a job share its W in one L2.
+  __shared__ ShortLds<D, IO> lds;
+  int q = static_cast<int>(blockIdx.x & 7) * (a.padded_items >> 3) + static_cast<int>(blockIdx.x >> 3);
+  if (q >= a.total_items) return;
+  int c = 0;
+  while (c + 1 < a.ncls && q >= a.cls_item_begin[c + 1]) ++c;
+  q -= a.cls_item_begin[c];
+  const int nch = a.cls_nchunks[c];
+  const int job = a.cls_job_begin[c] + q / nch;
+  const int lo = a.cls_tok_first[c] + q % nch * a.chunk;
+  const int hi = min(lo + a.chunk, a.cls_tok_first[c] + a.cls_tok_count[c]);
+  if ((cload(reinterpret_cast<const int*>(a.jobs + job) + 1) & 0xff) == CB_KIND_K) short_run<D, IO, true>(a, lds, job, lo, hi);
+  else short_run<D, IO, false>(a, lds, job, lo, hi);
 }
 
 // ---------------------------------------------------------------------------
@@ -2923,6 +3140,7 @@ struct cb_plan {
   int cls_unit_begin[kMaxClasses] = {0, 0, 0, 0};
   int cls_unit_end[kMaxClasses] = {0, 0, 0, 0};
   int cls_val_begin[kMaxClasses] = {0, 0, 0, 0};  // general kernel: first values unit
+  int cls_job_begin[kMaxClasses] = {0, 0, 0, 0}, cls_jobs[kMaxClasses] = {0, 0, 0, 0};
   int max_src_layer = 0, min_src_head = 0, max_src_head = 0;
   int max_tgt_layer = 0, min_tgt_head = 0, max_tgt_head = 0;
   void* d_w = nullptr;
@@ -3105,6 +3323,8 @@ int plan_build(const cb_plan_desc* d, const std::vector<int>& order, const std::
     int u = p->cls_unit_begin[c];
     while (u < p->cls_unit_end[c] && (jobs[unit_job[u]].y & 0xff) == CB_KIND_K) ++u;
     p->cls_val_begin[c] = u;
+    for (int v = p->cls_unit_begin[c]; v < p->cls_unit_end[c]; ++v) p->cls_jobs[c] += unit_njobs[v];
+    if (p->cls_jobs[c] > 0) p->cls_job_begin[c] = unit_job[p->cls_unit_begin[c]];
   }
   if (p->support_gemm) {
     // The support kernel gives XCD x units x, x + 8, ... of each class. Place
@@ -3473,6 +3693,30 @@ void split_cost_line(const cb_plan* p, MapArgs* a, bool allow_pool) {
   a->pool_gs = static_cast<int32_t>(gs);
 }
 
+// Tokens per workgroup of the short-request kernel, or 0 where the streaming
+// kernel is the faster one. The streaming kernel pays about 11 us and the
+// staging of every unit's W once, then less per token (its gather serves two
+// jobs), so the line moves with the jobs a CU has to map. Measured on MI355X
+// (streaming / short, us): 256 jobs, 64 tokens 12.8 / 8.3, 256 tokens 19.2 /
+// 18.0, 384 tokens 25.7 / 25.5; 1024 jobs, 64 tokens 35.0 / 25.0, 128 tokens
+// 40.2 / 36.6, 256 tokens 48.4 / 54.9; 1984 jobs, 64 tokens 58 / 41, 128
+// tokens 66 / 61; 48 fp32 jobs at D 64, 256 tokens 10.3 / 6.5, 1000 tokens
+// 14.1 / 11.3. Chunks keep two workgroups per CU busy: at 256 jobs, 128 tokens
+// take 11.6 us in two chunks and 12.4 in one, 256 tokens 18.0 in two and 20.0
+// in four.
+int short_chunk(const cb_plan* p, const int64_t* count) {
+  int64_t jobs = 0, job_tokens = 0, most = 0;
+  for (int c = 0; c < p->num_windows; ++c) {
+    jobs += p->cls_jobs[c];
+    job_tokens += p->cls_jobs[c] * count[c];
+    most = std::max(most, count[c]);
+  }
+  if (job_tokens > 112 * jobs + 256 * static_cast<int64_t>(p->num_cus)) return 0;
+  const int64_t chunks = std::max<int64_t>(1, 2 * static_cast<int64_t>(p->num_cus) / std::max<int64_t>(jobs, 1));
+  const int64_t tokens = (most + chunks - 1) / chunks;
+  return static_cast<int>(std::max<int64_t>(1, (tokens + kRoundTokens - 1) / kRoundTokens) * kRoundTokens);
+}
+
 template <typename IO>
 void launch_any(int D, int64_t items, hipStream_t s, const MapArgs& a) {
   const AnyShape sh = any_shape(D, sizeof(IO) == 4);
@@ -3502,6 +3746,9 @@ int launch_map(const cb_plan* p, MapArgs& a, const int64_t* first, const int64_t
   // The support kernel's items are fixed 256-token blocks; the knob does not apply.
   if (p->support_gemm) chunk = kSupTile;
   if (p->generic) chunk = std::min(chunk, any_tokens(any_shape(D, p->elem_bytes == 4).waves));
+  // An explicit tokens_per_workgroup is the streaming kernel's.
+  const int brief = ws && tokens_per_workgroup == 0 ? short_chunk(p, count) : 0;
+  if (brief) chunk = brief;
   a.w = static_cast<const uint4*>(p->d_w);
   a.bias = p->d_bias;
   a.wscale = p->d_scale;
@@ -3531,11 +3778,12 @@ int launch_map(const cb_plan* p, MapArgs& a, const int64_t* first, const int64_t
     a.cls_unit_begin[c] = p->cls_unit_begin[c];
     a.cls_unit_end[c] = p->cls_unit_end[c];
     a.cls_val_begin[c] = p->cls_val_begin[c];
+    a.cls_job_begin[c] = p->cls_job_begin[c];
     a.cls_tok_first[c] = static_cast<int32_t>(first[c]);
     a.cls_tok_count[c] = static_cast<int32_t>(count[c]);
     a.cls_nchunks[c] = static_cast<int32_t>(std::max<int64_t>(nch, 1));
     a.cls_item_begin[c] = static_cast<int32_t>(items);
-    items += static_cast<int64_t>(p->cls_unit_end[c] - p->cls_unit_begin[c]) * nch;
+    items += static_cast<int64_t>(brief ? p->cls_jobs[c] : p->cls_unit_end[c] - p->cls_unit_begin[c]) * nch;
     n_total = std::max(n_total, first[c] + count[c]);
   }
   a.n_tokens = static_cast<int32_t>(n_total);
@@ -3547,6 +3795,16 @@ int launch_map(const cb_plan* p, MapArgs& a, const int64_t* first, const int64_t
   int64_t grid_blocks = a.padded_items;
   if (p->generic)  // persistent: one workgroup of 8 waves per CU, or two of 4
     grid_blocks = std::min<int64_t>(grid_blocks, static_cast<int64_t>(p->num_cus) * (8 / any_shape(D, p->elem_bytes == 4).waves));
+  if (brief) {
+    const dim3 g(static_cast<unsigned>(grid_blocks)), b(kThreads);
+    p->last_pool_chunks.store(0, std::memory_order_relaxed);
+    p->last_workgroups.store(static_cast<int32_t>(g.x), std::memory_order_relaxed);
+    if (D == 128) hipLaunchKernelGGL((map_install_short_kernel<128, uint16_t>), g, b, 0, s, a);
+    else if (p->ntw == 2) hipLaunchKernelGGL((map_install_short_kernel<64, uint16_t>), g, b, 0, s, a);
+    else hipLaunchKernelGGL((map_install_short_kernel<64, float>), g, b, 0, s, a);
+    CB_HIP(hipGetLastError());
+    return CB_OK;
+  }
   // Held from the cost-line split through the launch and its pair event.
   std::unique_lock<std::mutex> held;
   int tracked_pair = -1;

@@ -158,7 +158,8 @@ typedef struct cb_request {
      generic kernels; the support kernel (support > 1 at head_dim 128, bf16)
      ignores it. For the streaming kernel a cap below the default shrinks the
      grid to about (tokens x units) / cap workgroups, which can make each
-     workgroup's share long enough for the work pool. */
+     workgroup's share long enough for the work pool; any cap keeps a short
+     request, which otherwise takes a kernel of its own, on this kernel. */
   int32_t tokens_per_workgroup;
 } cb_request;
 

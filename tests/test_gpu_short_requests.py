@@ -1,0 +1,93 @@
+"""GPU: short requests take a kernel of their own whose rows are bit-identical.
+
+The streaming kernel (forced by an explicit ``tokens_per_workgroup``) and the
+short-request kernel (the default at these lengths) must write the same bits:
+at the edges of the 16-token sub-tiles, 64-token rounds and workgroup chunks,
+with windows, per-layer thetas, slot vectors, batches and rows out of range.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from cachebridge_amd import synthetic
+from cachebridge_amd.online.blocks import map_install_batch, map_install_block
+from cachebridge_amd.plan import RequestSpan
+
+pytestmark = pytest.mark.gpu
+
+
+def _handoff(dim, dtype, tokens, windows=None, target_theta=1e6):
+    lt = 5
+    sh = synthetic.Shape(f"short{dim}", 6, 3, lt, 3, dim, tokens, dtype, [0, 2, 3, 5], source_theta=1e6,
+                         target_theta=target_theta, windows=windows, target_pages=2 * (tokens // 16 + 2), seed=31 + dim)
+    return synthetic.make_handoff(sh, fill_target="zeros")
+
+
+def _pools(h, run):
+    pool = h.target_pool
+    pool.k_data.fill_(0.25)
+    pool.v_data.fill_(0.25)
+    run()
+    torch.cuda.synchronize()
+    assert h.mapper.plan.read_errors() == 0
+    return pool.k_data.clone(), pool.v_data.clone()
+
+
+@pytest.mark.parametrize("dim,dtype", [(128, torch.bfloat16), (64, torch.bfloat16), (64, torch.float32)])
+@pytest.mark.parametrize("tokens", [1, 15, 16, 17, 63, 64, 65, 127, 129, 513, 700])
+def test_short_rows_equal_streaming_rows(dim, dtype, tokens):
+    print(f"short D={dim} {dtype} T={tokens}", flush=True)
+    windows = [None, 40, None, 40, 2] if tokens % 2 else None
+    h = _handoff(dim, dtype, tokens, windows, [1e6, 1e4, 1e6, 1e4, 1e6])
+    short = _pools(h, h.run)
+    chunks, groups = h.mapper.plan.last_split()
+    assert chunks == 0
+    stream = _pools(h, lambda: h.run(tokens_per_workgroup=512))
+    assert torch.equal(short[0], stream[0]) and torch.equal(short[1], stream[1])
+    assert bool((short[0] != 0.25).any())
+
+
+def test_short_batch_equals_per_request_rows():
+    """Ragged requests (one empty, one inside its prefix) in one short launch."""
+    print("short batch", flush=True)
+    lengths, starts = [37, 0, 16, 90], [0, 0, 100, 7]
+    h = _handoff(128, torch.bfloat16, sum(lengths), [None, 40, None, 40, 2])
+    need = [(n + 15) // 16 for n in lengths]
+    bt = torch.randperm(h.target_pool.pages, generator=torch.Generator().manual_seed(3))[:sum(need)].to(torch.int32).cuda()
+    spans, off, entry = [], 0, 0
+    for n, p, k in zip(lengths, starts, need):
+        spans.append(RequestSpan(off, entry * 16, n, p, 0))
+        off, entry = off + n, entry + k
+
+    def each():
+        for sp, k in zip(spans, need):
+            if sp.num_tokens:
+                map_install_batch(h.mapper, h.source_pool, h.source_slots, h.target_pool, [sp], block_table=bt, page_size=16)
+
+    got = _pools(h, lambda: map_install_batch(h.mapper, h.source_pool, h.source_slots, h.target_pool, spans,
+                                              block_table=bt, page_size=16))
+    want = _pools(h, each)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+def test_rows_out_of_range_are_flagged_not_written():
+    print("short rows out of range", flush=True)
+    h = _handoff(128, torch.bfloat16, 50)
+    slots = torch.arange(50, dtype=torch.int64, device="cuda")
+    good = _pools(h, lambda: map_install_block(h.mapper, h.source_pool, h.source_slots, h.target_pool, start=0, stop=50,
+                                               target_indices=slots))
+    bad_slots, bad_source = slots.clone(), h.source_slots.clone()
+    bad_slots[3] = h.target_pool.size
+    bad_slots[40] = -1
+    bad_source[20] = h.source_pool.size
+    pool = h.target_pool
+    pool.k_data.fill_(0.25)
+    pool.v_data.fill_(0.25)
+    map_install_block(h.mapper, h.source_pool, bad_source, pool, start=0, stop=50, target_indices=bad_slots)
+    assert h.mapper.plan.read_errors() == 3
+    for got, want in zip((pool.k_data, pool.v_data), good):
+        want = want.clone()
+        want[:, [3, 20, 40]] = 0.25
+        assert torch.equal(got, want)

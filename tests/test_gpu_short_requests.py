@@ -91,3 +91,35 @@ def test_rows_out_of_range_are_flagged_not_written():
         want = want.clone()
         want[:, [3, 20, 40]] = 0.25
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("windows", [None, [None, 300, None, 40, 2]])
+def test_support_rows_do_not_depend_on_the_request_length(windows):
+    """Support maps: waves without tokens, last blocks of every wave count and
+    unequal token chunks per job, against the rows of one long request."""
+    print(f"support lengths windows={windows}", flush=True)
+    sh = synthetic.Shape("support_lengths", 9, 3, 5, 3, 128, 700, torch.bfloat16, [], target_theta=1e6,
+                         windows=windows, head_map="identity", target_pages=128, seed=41, support=4)
+    h = synthetic.make_handoff(sh, fill_target="zeros")
+    pool = h.target_pool
+    slots = torch.randperm(pool.size, generator=torch.Generator().manual_seed(2))[:700].cuda()
+
+    def rows(start, stop):
+        pool.k_data.fill_(0.25)
+        pool.v_data.fill_(0.25)
+        map_install_block(h.mapper, h.source_pool, h.source_slots, pool, start=start, stop=stop, target_indices=slots,
+                          prefix_length=700)
+        torch.cuda.synchronize()
+        assert h.mapper.plan.read_errors() == 0
+        return pool.k_data[:, slots].clone(), pool.v_data[:, slots].clone(), pool.k_data.clone()
+
+    whole = rows(0, 700)
+    for start, n in [(0, 1), (0, 31), (5, 32), (0, 33), (0, 96), (400, 224), (400, 225), (400, 256), (0, 257), (389, 311),
+                     (100, 513)]:
+        got = rows(start, start + n)
+        for a, b in zip(got[:2], whole[:2]):
+            assert torch.equal(a[:, start:start + n], b[:, start:start + n]), (start, n)
+            assert bool((a[:, :start] == 0.25).all()) and bool((a[:, start + n:] == 0.25).all()), (start, n)
+        outside = torch.ones(pool.size, dtype=torch.bool, device="cuda")
+        outside[slots] = False
+        assert bool((got[2][:, outside] == 0.25).all())

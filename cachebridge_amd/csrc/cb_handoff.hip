@@ -358,10 +358,6 @@ struct MapArgs {
   int32_t cls_subtiles[kMaxClasses];     // 16-token sub-tiles of each class's tokens
   int32_t num_units;
   int32_t num_blocks;
-  // Range r of the cost line covers (unit, sub-tile) from blk_unit/sub[r] to
-  // blk_unit/sub[r + 1] (cut on the host, split_cost_line).
-  int32_t blk_unit[kMaxStreamBlocks + 1];
-  int32_t blk_sub[kMaxStreamBlocks + 1];
   int32_t* err;
   void* sink;  // scratch destination of stores without a target row
   const void* zero;  // one all-zero head row: the gather source of tokens without a source row
@@ -378,6 +374,15 @@ struct MapArgs {
   int32_t pool_u0;
   int32_t pool_s0;
   int32_t pool_gs;
+};
+
+// The streaming kernel's arguments (the other kernels' are a quarter of their
+// size, which every launch copies).
+struct StreamArgs : MapArgs {
+  // Range r of the cost line covers (unit, sub-tile) from blk_unit/sub[r] to
+  // blk_unit/sub[r + 1] (cut on the host, split_cost_line).
+  int32_t blk_unit[kMaxStreamBlocks + 1];
+  int32_t blk_sub[kMaxStreamBlocks + 1];
 };
 
 // Job flag (meta.z): un-rotation uses the rotation table (same theta, unit norm).
@@ -419,7 +424,7 @@ __device__ inline bool decode_work(const MapArgs& a, Work* w) {
 struct Pos {
   int unit, sub;
 };
-static_assert(sizeof(MapArgs) <= 4096, "kernel arguments must fit 4 KB");
+static_assert(sizeof(StreamArgs) <= 4096, "kernel arguments must fit 4 KB");
 
 // Position of token t of the launch (see MapArgs::pos).
 __device__ inline int position_of(const MapArgs& a, int t) {
@@ -944,7 +949,7 @@ __device__ void stream_run(const MapArgs& a, uint4* lds_w, float* lds_bias, int*
 }
 
 template <int D, typename IO, bool POS>
-__global__ __launch_bounds__(kStreamThreads) void map_install_stream_kernel(MapArgs a) {
+__global__ __launch_bounds__(kStreamThreads) void map_install_stream_kernel(StreamArgs a) {
   __shared__ uint4 lds_w[kUnitJobs * Gm<D, IO>::W_U4];
   __shared__ float lds_bias[kUnitJobs * D];
   __shared__ int lds_next;  // next sub-tile to claim in the current segment
@@ -3639,7 +3644,7 @@ constexpr int64_t kSegmentCost = 256;
 // budget), so ranges that cross a unit boundary get fewer sub-tiles. With a
 // work pool, the ranges are filled to a smaller budget and the rest of the
 // line becomes the pool (a->pool_*).
-void split_cost_line(const cb_plan* p, MapArgs* a, bool allow_pool) {
+void split_cost_line(const cb_plan* p, StreamArgs* a, bool allow_pool) {
   const int nu = p->num_units, nb = a->num_blocks;
   std::vector<int32_t> ns(nu, 0);
   int64_t total = 0;
@@ -3785,7 +3790,7 @@ void launch_any(int D, int64_t items, hipStream_t s, const MapArgs& a) {
 // count[c]) of the launch's token space. `a` carries the two sides (and, for
 // batches, the position vector); the plan fields are filled in here.
 // tokens_per_workgroup > 0 caps the unit-tokens per workgroup.
-int launch_map(const cb_plan* p, MapArgs& a, const int64_t* first, const int64_t* count,
+int launch_map(const cb_plan* p, StreamArgs& a, const int64_t* first, const int64_t* count,
                int tokens_per_workgroup, int default_tokens, hipStream_t s) {
   const int D = p->info.head_dim;
   const bool ws = p->info.support == 1 && !p->generic;
@@ -3797,6 +3802,7 @@ int launch_map(const cb_plan* p, MapArgs& a, const int64_t* first, const int64_t
   if (p->support_gemm) chunk = kSupTile;
   if (p->generic) chunk = std::min(chunk, any_tokens(any_shape(D, p->elem_bytes == 4).waves));
   // An explicit tokens_per_workgroup is the streaming kernel's.
+  const MapArgs& base = a;
   const int brief = ws && tokens_per_workgroup == 0 ? short_chunk(p, count) : 0;
   if (brief) chunk = brief;
   a.w = static_cast<const uint4*>(p->d_w);
@@ -3849,9 +3855,9 @@ int launch_map(const cb_plan* p, MapArgs& a, const int64_t* first, const int64_t
     const dim3 g(static_cast<unsigned>(grid_blocks)), b(kThreads);
     p->last_pool_chunks.store(0, std::memory_order_relaxed);
     p->last_workgroups.store(static_cast<int32_t>(g.x), std::memory_order_relaxed);
-    if (D == 128) hipLaunchKernelGGL((map_install_short_kernel<128, uint16_t>), g, b, 0, s, a);
-    else if (p->ntw == 2) hipLaunchKernelGGL((map_install_short_kernel<64, uint16_t>), g, b, 0, s, a);
-    else hipLaunchKernelGGL((map_install_short_kernel<64, float>), g, b, 0, s, a);
+    if (D == 128) hipLaunchKernelGGL((map_install_short_kernel<128, uint16_t>), g, b, 0, s, base);
+    else if (p->ntw == 2) hipLaunchKernelGGL((map_install_short_kernel<64, uint16_t>), g, b, 0, s, base);
+    else hipLaunchKernelGGL((map_install_short_kernel<64, float>), g, b, 0, s, base);
     CB_HIP(hipGetLastError());
     return CB_OK;
   }
@@ -3960,15 +3966,15 @@ int launch_map(const cb_plan* p, MapArgs& a, const int64_t* first, const int64_t
       const int64_t last = count[c] % kSupTile;
       idle = idle || (last > 0 && last <= kSupTile - 32 && count[c] <= 4 * kSupTile);
     }
-    if (idle) hipLaunchKernelGGL(map_install_support_kernel<true>, dim3(8 * per_xcd), dim3(kSupThreads), 0, s, a);
-    else hipLaunchKernelGGL(map_install_support_kernel<false>, dim3(8 * per_xcd), dim3(kSupThreads), 0, s, a);
+    if (idle) hipLaunchKernelGGL(map_install_support_kernel<true>, dim3(8 * per_xcd), dim3(kSupThreads), 0, s, base);
+    else hipLaunchKernelGGL(map_install_support_kernel<false>, dim3(8 * per_xcd), dim3(kSupThreads), 0, s, base);
   } else {
     if (D == 128 && p->ntw == 2)
-      hipLaunchKernelGGL((map_install_gen_kernel<128, uint16_t>), grid, block, 0, s, a);
+      hipLaunchKernelGGL((map_install_gen_kernel<128, uint16_t>), grid, block, 0, s, base);
     else if (D == 64 && p->ntw == 2)
-      hipLaunchKernelGGL((map_install_gen_kernel<64, uint16_t>), grid, block, 0, s, a);
+      hipLaunchKernelGGL((map_install_gen_kernel<64, uint16_t>), grid, block, 0, s, base);
     else
-      hipLaunchKernelGGL((map_install_gen_kernel<64, float>), grid, block, 0, s, a);
+      hipLaunchKernelGGL((map_install_gen_kernel<64, float>), grid, block, 0, s, base);
   }
   CB_HIP(hipGetLastError());
   return CB_OK;
@@ -4206,7 +4212,7 @@ int cb_map_install(const cb_plan* p, const cb_request* rq, void* stream) {
   const cb_rows& tr = rq->target;
   int rc;
   if ((rc = check_sides(p, sr, tr))) return rc;
-  MapArgs a{};
+  StreamArgs a{};
   const int align = p->generic ? p->elem_bytes : 16;
   if ((rc = to_dev_rows(sr, p->elem_bytes, &a.src, align))) return rc;
   if ((rc = to_dev_rows(tr, p->elem_bytes, &a.tgt, align))) return rc;
@@ -4290,7 +4296,7 @@ int cb_map_install_batch(const cb_plan* p, const cb_rows* source, const cb_rows*
   }
   // The map launch reads the resolved rows as int32 row vectors over the
   // batch's token space, and each key token's position from the third section.
-  MapArgs a{};
+  StreamArgs a{};
   a.src = b.src;
   a.tgt = b.tgt;
   for (DevRows* side : {&a.src, &a.tgt}) {

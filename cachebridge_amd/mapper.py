@@ -82,6 +82,7 @@ class HeadwiseMapper:
         if len(windows) != lt:
             raise ValueError("windows needs one entry per target layer")
         self.windows = windows
+        self._windowed = any(w is not None for w in windows)
         theta_sets: list[ThetaSet] = []
 
         def theta_index(ts: ThetaSet) -> int:
@@ -207,7 +208,7 @@ class HeadwiseMapper:
                 raise ValueError("preallocated mapper output geometry/dtype/device mismatch")
         direct = output is not None and output.device == self.device and output.is_contiguous()
         out = output if direct else torch.empty(expected, dtype=self.dtype, device=self.device)
-        if any(w is not None for w in self.windows):
+        if self._windowed:
             # Window-excluded tokens of a dense output are not computed; define them.
             out.zero_()
         self.plan.launch(rows_from_page(page, head_offset=source_head_offset), rows_from_page(out),

@@ -111,7 +111,6 @@ def map_write_block(mapper, block, target_pool, target_indices, *, start, source
     mapper.map_install(source, target, num_tokens=n, position_start=start)
 
 
-@torch.inference_mode()
 def map_install_block(mapper, source_pool, source_indices, target_pool, *, start, stop,
                       target_indices=None, block_table=None, page_size=None,
                       source_head_offset=0, prefix_length=0, stream=None,

@@ -93,16 +93,10 @@ def rows_from_page(page: torch.Tensor, *, head_offset: int = 0, tokens=None) -> 
     if not page.is_contiguous():
         raise ValueError("page must be contiguous")
     _, layers, n, heads, dim = page.shape
-    c = _lib.CbRows()
-    c.k_base = page[0].data_ptr()
-    c.v_base = page[1].data_ptr()
-    c.layer_stride = n * heads * dim
-    c.row_stride = heads * dim
-    c.rows = n
-    c.num_layers = layers
-    c.head_offset = head_offset
-    c.heads = heads
-    c.index_kind = _lib.CB_INDEX_IDENTITY
+    base = page.data_ptr()
+    plane = n * heads * dim
+    c = _lib.CbRows(None, None, base, base + layers * plane * page.element_size() if base else 0, plane, heads * dim,
+                    n, layers, head_offset, heads, _lib.CB_INDEX_IDENTITY)
     return Rows(c, page.dtype, page.device, [page])
 
 
@@ -161,19 +155,8 @@ def rows_from_stacked(k: torch.Tensor, v: torch.Tensor, *, index=None, block_tab
         raise ValueError("stacked K/V must be contiguous")
     layers, rows, heads, dim = k.shape
     kind, idx_ptr, keep = _index_fields(index, block_table, page_size, index_offset, tokens)
-    c = _lib.CbRows()
-    c.k_base = k.data_ptr()
-    c.v_base = v.data_ptr()
-    c.layer_stride = rows * heads * dim
-    c.row_stride = heads * dim
-    c.rows = rows
-    c.num_layers = layers
-    c.head_offset = head_offset
-    c.heads = heads
-    c.index_kind = kind
-    c.index = idx_ptr
-    c.index_offset = index_offset
-    c.page_size = page_size or 0
+    c = _lib.CbRows(None, None, k.data_ptr(), v.data_ptr(), rows * heads * dim, heads * dim, rows, layers, head_offset,
+                    heads, kind, idx_ptr, index_offset, page_size or 0)
     return Rows(c, k.dtype, k.device, [k, v, *keep])
 
 
@@ -341,13 +324,8 @@ class HandoffPlan:
             raise ValueError(f"source/target dtype must be {self.dtype}")
         if source.device != self.device or target.device != self.device:
             raise ValueError("source, target and plan must be on the same device")
-        req = _lib.CbRequest()
-        req.source = source.c
-        req.target = target.c
-        req.num_tokens = int(num_tokens)
-        req.position_start = int(position_start)
-        req.prefix_length = int(prefix_length)
-        req.tokens_per_workgroup = int(tokens_per_workgroup)
+        req = _lib.CbRequest(source.c, target.c, int(num_tokens), int(position_start), int(prefix_length),
+                             int(tokens_per_workgroup))
         _lib.check(self.lib.cb_map_install(self._handle, ctypes.byref(req),
                                            _lib.stream_handle(stream)))
         source.hold_for(stream)

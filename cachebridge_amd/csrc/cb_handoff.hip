@@ -3113,6 +3113,126 @@ __global__ __launch_bounds__(512, 2) void delta_state128_kernel(DeltaArgs p) {
     for (int e = 0; e < 4; ++e) out[(16 * w + 4 * q + e) * kDs + 16 * jb + r] = oo[jb][e];
 }
 
+// fp32 states whose value dimensions are 64, 128 or 256 (16 NV, 16 NO), output
+// key dimension 64 or 128 and key dimension a multiple of 32: a workgroup of W
+// waves per batch entry and 16 W rows of T and of out, wave w owning 16 of
+// them. The general kernel reads every operand of its MFMAs from global memory
+// and forms 16 rows a workgroup; staging and 64 or 128 rows took 384 states of
+// 128 x 256 -> 128 x 256 from 747 to 125 us, of 64 x 64 from 21.0 to 7.9
+// (bound by the fp32 MFMAs, 103 TFLOP/s of 157, at the larger).
+//   Stage 1 forms T^T = U^T A as 16x16 tiles (v-block vb, row block w): A
+//   operand U[k][16vb + r], B operand A[k][16w + r], over 32-row chunks of A
+//   and U staged through LDS (double-buffered; the next chunk's loads are in
+//   flight during the current chunk's MFMAs).
+//   Stage 2 uses those accumulators directly as the A operand of out = T B:
+//   lane (q, r) of tile vb holds T[16w + r][16vb + 4q + e], so k-step (vb, e)
+//   pairs lane q with row 16vb + 4q + e of B (a permuted k order; the sum over
+//   v is the same). B streams through the same LDS buffers.
+// Chunk rows are padded by 16 floats (rows q, q + 1 of a k-step) for A and U
+// and by 4 for B (rows 4q, 4q + 4), so every operand read hits 64 banks.
+template <int W, int NV, int NO>
+struct DeltaTile {
+  static constexpr int V = 16 * NV, VP = 16 * NO, KP = 16 * W;
+  static constexpr int SA = KP + 16, SU = V + 16, SB = VP + 4;      // LDS row strides (floats)
+  static constexpr int kStage1 = kDsChunk * (SA + SU);              // floats per buffer
+  static constexpr int kStage2 = kDsChunk * SB;
+  static constexpr int kBuf = kStage1 > kStage2 ? kStage1 : kStage2;
+};
+
+template <int W, int NV, int NO>
+__global__ __launch_bounds__(W * kWave, 2) void delta_tile_kernel(DeltaArgs p) {
+  using C = DeltaTile<W, NV, NO>;
+  constexpr int NT = W * kWave;
+  __shared__ float lds[2 * C::kBuf];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int64_t bi = blockIdx.x;
+  const float* U = static_cast<const float*>(p.u) + bi * p.su;
+  const float* A = static_cast<const float*>(p.a) + bi * p.sa + blockIdx.y * C::KP;  // this workgroup's columns
+  const float* B = static_cast<const float*>(p.b) + bi * p.sb;
+  float* out = static_cast<float*>(p.out) + bi * p.so + static_cast<int64_t>(blockIdx.y) * C::KP * C::VP;
+  // COLS columns of a 32-row chunk, rows `ld` apart: 16 bytes per thread and step.
+  auto load_chunk = [&](const float* m, int ld, auto colsc, int c, f32x4* v) __attribute__((always_inline)) {
+    constexpr int COLS = decltype(colsc)::value, N = kDsChunk * COLS / 4 / NT;
+    static_assert(kDsChunk * COLS / 4 % NT == 0, "chunk split");
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int at = (i * NT + threadIdx.x) * 4;
+      v[i] = *reinterpret_cast<const f32x4*>(m + (static_cast<int64_t>(c) * kDsChunk + at / COLS) * ld + at % COLS);
+    }
+  };
+  auto store_chunk = [&](float* dst, auto colsc, auto stridec, const f32x4* v) __attribute__((always_inline)) {
+    constexpr int COLS = decltype(colsc)::value, S = decltype(stridec)::value, N = kDsChunk * COLS / 4 / NT;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int at = (i * NT + threadIdx.x) * 4;
+      *reinterpret_cast<f32x4*>(dst + at / COLS * S + at % COLS) = v[i];
+    }
+  };
+  constexpr std::integral_constant<int, C::KP> ca{};
+  constexpr std::integral_constant<int, C::V> cu{};
+  constexpr std::integral_constant<int, C::VP> cb{};
+  constexpr std::integral_constant<int, C::SA> sa{};
+  constexpr std::integral_constant<int, C::SU> su{};
+  constexpr std::integral_constant<int, C::SB> sb{};
+  f32x4 av[kDsChunk * C::KP / 4 / NT], uv[kDsChunk * C::V / 4 / NT], bv[kDsChunk * C::VP / 4 / NT];
+
+  // Stage 1: tt[vb] = (U^T A) tile (vb, w), i.e. T[16w + r][16vb + 4q + e].
+  f32x4 tt[NV];
+#pragma unroll
+  for (int vb = 0; vb < NV; ++vb) tt[vb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int nk = p.k / kDsChunk;
+  load_chunk(A, p.kp, ca, 0, av);
+  load_chunk(U, C::V, cu, 0, uv);
+  load_chunk(B, C::VP, cb, 0, bv);
+  for (int c = 0; c < nk; ++c) {
+    float* bufA = lds + (c & 1) * C::kBuf;
+    float* bufU = bufA + kDsChunk * C::SA;
+    store_chunk(bufA, ca, sa, av);
+    store_chunk(bufU, cu, su, uv);
+    __syncthreads();
+    const int cn = c + 1 < nk ? c + 1 : c;  // (the last chunk again at the end: no branch around the loads)
+    load_chunk(A, p.kp, ca, cn, av);
+    load_chunk(U, C::V, cu, cn, uv);
+#pragma unroll
+    for (int kk = 0; kk < kDsChunk; kk += 4) {
+      const float x = bufA[(kk + q) * C::SA + 16 * w + r];
+#pragma unroll
+      for (int vb = 0; vb < NV; ++vb)
+        tt[vb] = __builtin_amdgcn_mfma_f32_16x16x4f32(bufU[(kk + q) * C::SU + 16 * vb + r], x, tt[vb], 0, 0, 0);
+    }
+  }
+
+  // Stage 2: oo[jb] = out tile (w, jb) = sum over v of T[16w + .][v] B[v][16jb + .].
+  f32x4 oo[NO];
+#pragma unroll
+  for (int jb = 0; jb < NO; ++jb) oo[jb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // (The first B chunk goes into the buffer that stage 1's last chunk leaves free.)
+#pragma unroll
+  for (int c = 0; c < NV / 2; ++c) {
+    float* bufB = lds + ((nk + c) & 1) * C::kBuf;
+    store_chunk(bufB, cb, sb, bv);
+    __syncthreads();
+    if (c + 1 < NV / 2) load_chunk(B, C::VP, cb, c + 1, bv);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {        // v-blocks 2c, 2c + 1 of this chunk
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int vrow = 16 * h + 4 * q + e;
+        const float x = tt[2 * c + h][e];  // c and h are unrolled constants
+#pragma unroll
+        for (int jb = 0; jb < NO; ++jb)
+          oo[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, bufB[vrow * C::SB + 16 * jb + r], oo[jb], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int jb = 0; jb < NO; ++jb)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[static_cast<int64_t>(16 * w + 4 * q + e) * C::VP + 16 * jb + r] = oo[jb][e];
+}
+
 // ---------------------------------------------------------------------------
 // Batched launches: every kept token of every request gets a slot in one
 // token space, class by class (class c's kept tokens of request r occupy
@@ -4060,6 +4180,37 @@ void* scratch_on(int device) {
   return g_scratch_ptr[device];
 }
 
+constexpr unsigned kDeltaSplitBatch = 128;
+
+// Whether delta_tile_kernel takes a transform: its dimensions, and 16-byte
+// aligned rows.
+bool delta_tiled(const DeltaArgs& a) {
+  const auto value_dim = [](int n) { return n == 64 || n == 128 || n == 256; };
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(a.u) | reinterpret_cast<uintptr_t>(a.a) | reinterpret_cast<uintptr_t>(a.b);
+  return a.k % kDsChunk == 0 && (a.kp == 64 || a.kp == 128) && value_dim(a.v) && value_dim(a.vp) && bits % 16 == 0 &&
+         (a.su | a.sa | a.sb) % 4 == 0;
+}
+
+template <int W, int NV>
+void launch_delta_out(const DeltaArgs& a, dim3 g, hipStream_t s) {
+  if (a.vp == 64) hipLaunchKernelGGL((delta_tile_kernel<W, NV, 4>), g, dim3(W * kWave), 0, s, a);
+  else if (a.vp == 128) hipLaunchKernelGGL((delta_tile_kernel<W, NV, 8>), g, dim3(W * kWave), 0, s, a);
+  else hipLaunchKernelGGL((delta_tile_kernel<W, NV, 16>), g, dim3(W * kWave), 0, s, a);
+}
+
+template <int W>
+void launch_delta_value(const DeltaArgs& a, dim3 g, hipStream_t s) {
+  if (a.v == 64) launch_delta_out<W, 4>(a, g, s);
+  else if (a.v == 128) launch_delta_out<W, 8>(a, g, s);
+  else launch_delta_out<W, 16>(a, g, s);
+}
+
+void launch_delta_tile(const DeltaArgs& a, unsigned batch, hipStream_t s) {
+  // 64 rows per workgroup where the batch alone leaves CUs idle.
+  if (a.kp == 64 || batch <= kDeltaSplitBatch) launch_delta_value<4>(a, dim3(batch, a.kp / 64), s);
+  else launch_delta_value<8>(a, dim3(batch), s);
+}
+
 }  // namespace
 
 extern "C" {
@@ -4393,7 +4544,9 @@ int cb_delta_state_transform(int32_t dtype, int64_t batch, int32_t k, int32_t v,
               k, v, kp, vp};
   const dim3 grid(static_cast<unsigned>(batch), static_cast<unsigned>((kp + 15) / 16));
   const bool square128 = k == kDs && v == kDs && kp == kDs && vp == kDs;
-  if (dtype == CB_DTYPE_F32 && square128)
+  if (dtype == CB_DTYPE_F32 && !square128 && delta_tiled(a)) {
+    launch_delta_tile(a, static_cast<unsigned>(batch), static_cast<hipStream_t>(stream));
+  } else if (dtype == CB_DTYPE_F32 && square128)
     hipLaunchKernelGGL(delta_state128_kernel, dim3(static_cast<unsigned>(batch)), dim3(512), 0,
                        static_cast<hipStream_t>(stream), a);
   else if (dtype == CB_DTYPE_F32)

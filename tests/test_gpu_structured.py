@@ -100,3 +100,24 @@ def test_empty_batch_and_limits():
     with pytest.raises(ValueError, match="dtype"):
         arch.transform_delta_state(torch.zeros(1, 4, 4, device="cuda"), torch.zeros(4, 3, device="cuda"),
                                    torch.zeros(4, 2, device="cuda", dtype=torch.float64))
+
+
+@pytest.mark.parametrize("batch", [3, 129])
+@pytest.mark.parametrize("k,v,kp,vp", [(32, 64, 64, 64), (96, 64, 128, 256), (64, 256, 64, 128), (128, 256, 128, 64),
+                                       (160, 128, 64, 256), (64, 128, 128, 128)])
+def test_tiled_dimensions_match_oracle(k, v, kp, vp, batch):
+    """Dimensions of the staged kernel, below and above the batch at which a
+    workgroup takes 128 rows, with a shared basis, and the same operands at
+    addresses that only the general kernel takes."""
+    print(f"delta tiles {batch}x k={k} v={v} kp={kp} vp={vp}", flush=True)
+    g = torch.Generator().manual_seed(k + v + kp + vp)
+    u = torch.randn(batch, k, v, generator=g)
+    a = torch.randn(k, kp, generator=g)
+    b = torch.randn(batch, v, vp, generator=g)
+    out = arch.transform_delta_state(u.cuda(), a.cuda(), b.cuda())
+    odd = torch.zeros(u.numel() + 1, device="cuda")
+    odd[1:] = u.reshape(-1).cuda()
+    general = arch.transform_delta_state(odd[1:].view(u.shape), a.cuda(), b.cuda())
+    torch.cuda.synchronize()
+    _check(out, u, a.expand(batch, k, kp), b)
+    _check(general, u, a.expand(batch, k, kp), b)

@@ -1779,17 +1779,18 @@ __global__ __launch_bounds__(kSupThreads, 1) void map_install_support_kernel(Map
   SupItems items;
   items.x = blockIdx.x & 7;
   items.nwg = gridDim.x >> 3;
-  // Turn by turn, workgroup i takes item i of the XCD's next nwg items, every
-  // second turn item nwg - 1 - i: where a job's token chunks differ in length
-  // (two chunks of 16 jobs make one turn of 32), a workgroup then gets one of
-  // each. Only the last turn can be short, so an item past the end ends the
+  // Turn by turn, workgroup i takes item i of the XCD's next nwg items; with
+  // short blocks about, every second turn item nwg - 1 - i: where a job's token
+  // chunks differ in length (two chunks of 16 jobs make one turn of 32), a
+  // workgroup then gets one of each. Only the last turn can be short, so an item past the end ends the
   // workgroup's list.
   items.next = blockIdx.x >> 3;
-  int step = 2 * (items.nwg - static_cast<int>(items.next)) - 1;  // to the mirrored item of the next turn
+  // (To the mirrored item of the next turn, or the same.)
+  int step = IDLE ? 2 * (items.nwg - static_cast<int>(items.next)) - 1 : items.nwg;
   uint32_t slot = 0;  // ring slot of the last stage run
   int errbits = 0;
   SupItems::Item it;
-  for (; items.get(a, it); items.next += step, step = 2 * items.nwg - step) {
+  for (; items.get(a, it); items.next += step, step = IDLE ? 2 * items.nwg - step : step) {
     SupLane I;
     I.job = __builtin_amdgcn_readfirstlane(it.job);
     if constexpr (IDLE) {
@@ -2787,7 +2788,7 @@ __global__ __launch_bounds__(NW * kWave, 2) void map_install_any_kernel(MapArgs 
 // Plan data of the general kernel: W in fragment order (any_w_offset, padded
 // entries zero), for fp16 with every output dim scaled by the power of two
 // that brings its largest weight into [2^13, 2^14), the inverse scales, and
-// the bias, in sorted job order. One workgroup per job.
+// the bias, in sorted job order. Grid: (jobs, shares of a job's entries).
 __global__ __launch_bounds__(256) void pack_any_kernel(const float* __restrict__ w, const float* __restrict__ bias,
                                                        const int32_t* __restrict__ order, int S, int D, int scaled,
                                                        float* __restrict__ wp, float* __restrict__ bp,
@@ -2807,15 +2808,17 @@ __global__ __launch_bounds__(256) void pack_any_kernel(const float* __restrict__
       }
     }
     scale[o] = sc;
+    if (blockIdx.y > 0) continue;
     sp[job * D + o] = 1.f / sc;
     bp[job * D + o] = bias[from * D + o];
   }
   __syncthreads();
-  const int Q = any_chunks(D), NG = any_groups(D), half = D / 2;
-  const int64_t total = static_cast<int64_t>(S) * Q * 2 * NG * kAnyFragU4 * 4;
+  const uint32_t Q = any_chunks(D), NG = any_groups(D);
+  const int half = D / 2;
+  const uint32_t total = S * Q * 2 * NG * kAnyFragU4 * 4;  // at most 2^24
   float* dst = wp + job * total;
-  for (int64_t idx = threadIdx.x; idx < total; idx += blockDim.x) {
-    int64_t rem = idx;
+  for (uint32_t idx = blockIdx.y * blockDim.x + threadIdx.x; idx < total; idx += gridDim.y * blockDim.x) {
+    uint32_t rem = idx;
     const int e0 = rem % 4; rem /= 4;
     const int lane = rem % kWave; rem /= kWave;
     const int e = e0 + 4 * static_cast<int>(rem % 2); rem /= 2;
@@ -3624,7 +3627,7 @@ int plan_build(const cb_plan_desc* d, const std::vector<int>& order, const std::
   if (e == hipSuccess) {
     uint16_t* wp = static_cast<uint16_t*>(p->d_w);
     if (p->generic)
-      hipLaunchKernelGGL(pack_any_kernel, dim3(nj), dim3(256), 0, 0, d->d_weight, d->d_bias, d_order, S, D,
+      hipLaunchKernelGGL(pack_any_kernel, dim3(nj, 8), dim3(256), 0, 0, d->d_weight, d->d_bias, d_order, S, D,
                          d->io_dtype == CB_DTYPE_F16 ? 1 : 0, static_cast<float*>(p->d_w), p->d_bias, p->d_scale);
     else if (D == 64 && p->ntw == 2)
       launch_pack<64, 2>(d, d_order, wp, p->d_bias);

@@ -2087,12 +2087,18 @@ __global__ void pack_weights_kernel(const float* __restrict__ w, const float* __
 // terms (24 bits; the products of terms i + j < 3: 6 for keys, 3 for values,
 // whose bf16 inputs are exact); fp16 into two fp16 terms of 11 bits each (3
 // and 2 products), with W scaled by a power of two per output dim at plan time
-// and keys by 1/2 (so that no finite input overflows); fp32 multiplies in
-// fp32, each part into accumulators of its own. The results are as close to
-// the 64-bit ones as those of fp32 fused multiply-adds (relative error at D
-// 256 bf16 1.658136e-3 with both, at D 128 fp16 2.07488e-4 and fp32 2.11e-7
-// with those, 2.07488e-4 and 1.57e-7 here; two bf16 terms gave 1.658142e-3).
-// An output that is not finite (an infinity or NaN in its source row) is
+// and keys by 4; fp32 multiplies in fp32, each part into accumulators of its
+// own. fp16 has few exponents: the second term of a small key would be a
+// subnormal, so it is kept times 2^11 (at most 2^15) and multiplied by W's
+// first term times 2^-11, which leaves a key an absolute error of 2^-38
+// instead of 2^-24.
+// Relative errors against 64 bits before the rounding to the pool's type (D
+// 128, keys N(0, 1) times 1 / 1e-2 / 1e-3 / 1e-4): fp32 fused multiply-adds
+// 2.0e-7 throughout, fp16 terms 1e-7 throughout (unscaled second terms: 1e-7 /
+// 3e-6 / 3e-5 / 3e-4). After it, at D 256 bf16 1.658136e-3 with both (two
+// bf16 terms: 1.658142e-3), at D 128 fp32 2.11e-7 with those, 1.57e-7 here.
+// An output that is not finite (an infinity or NaN in its source row, or an
+// fp16 key of 2^14 or more, whose scaled first term is infinite) is
 // computed again term by term in fp32, because an infinity times the terms of
 // a weight need not keep its sign.
 //
@@ -2136,19 +2142,22 @@ struct AnyIO<uint16_t> {  // bf16
   using Frag = bf16x8;
   static constexpr int kTerms = 3;
   static constexpr float kKeyScale = 1.f;
+  static constexpr float kLowScale = 1.f;
   static constexpr bool kScaled = false;
   static __device__ float get(const CB_GLOBAL uint16_t* p) { return bf2f(*p); }
   static __device__ uint16_t put(float v) { return f2bf(v); }
   static __device__ uint32_t pack(float a, float b) { return pack_bf16(a, b); }
   static __device__ float lo(uint32_t w) { return lo_bf(w); }
   static __device__ float hi(uint32_t w) { return hi_bf(w); }
+  static __device__ float rest(float v, float term, float) { return v - term; }
   static __device__ f32x4 mul(const Frag& a, const Frag& b, const f32x4& c) { return mfma(a, b, c); }
 };
 template <>
 struct AnyIO<_Float16> {
   using Frag = f16x8;
   static constexpr int kTerms = 2;
-  static constexpr float kKeyScale = 0.5f;
+  static constexpr float kKeyScale = 4.f;
+  static constexpr float kLowScale = 2048.f;  // of a key's second term
   static constexpr bool kScaled = true;  // weights scaled per output dim
   static __device__ float get(const CB_GLOBAL _Float16* p) { return static_cast<float>(*p); }
   static __device__ _Float16 put(float v) { return static_cast<_Float16>(v); }
@@ -2158,6 +2167,8 @@ struct AnyIO<_Float16> {
   }
   static __device__ float lo(uint32_t w) { return static_cast<float>(__builtin_bit_cast(f16x2, w)[0]); }
   static __device__ float hi(uint32_t w) { return static_cast<float>(__builtin_bit_cast(f16x2, w)[1]); }
+  // (v - term) * low, exact: one instruction that converts the term, one more for a low other than 1.
+  static __device__ float rest(float v, float term, float low) { return __builtin_fmaf(-term, low, v * low); }
   static __device__ f32x4 mul(const Frag& a, const Frag& b, const f32x4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
@@ -2172,17 +2183,19 @@ struct AnyIO<float> {
 };
 
 // Eight values as terms of the 16-bit type: each the rounded rest of those
-// before it, element pairs packed.
-template <typename IO>
+// before it (KEY: times kLowScale), element pairs packed.
+template <typename IO, bool KEY>
 __device__ __attribute__((always_inline)) inline void any_split(const float (&v)[8], uint32_t (&h)[AnyIO<IO>::kTerms][4]) {
+  constexpr float low = KEY ? AnyIO<IO>::kLowScale : 1.f;
+  static_assert(low == 1.f || AnyIO<IO>::kTerms == 2, "one scaled term");
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     float a = v[2 * e], b = v[2 * e + 1];
 #pragma unroll
     for (int t = 0; t < AnyIO<IO>::kTerms; ++t) {
       h[t][e] = AnyIO<IO>::pack(a, b);
-      a = a - AnyIO<IO>::lo(h[t][e]);
-      b = b - AnyIO<IO>::hi(h[t][e]);
+      a = AnyIO<IO>::rest(a, AnyIO<IO>::lo(h[t][e]), low);
+      b = AnyIO<IO>::rest(b, AnyIO<IO>::hi(h[t][e]), low);
     }
   }
 }
@@ -2431,8 +2444,8 @@ __device__ __attribute__((always_inline)) inline void any_run(const MapArgs& a, 
         }
       } else {
         uint32_t h[2][WT][4];  // [part][term][element pair]
-        any_split<IO>(k1, h[0]);
-        any_split<IO>(k2, h[1]);
+        any_split<IO, true>(k1, h[0]);
+        any_split<IO, true>(k2, h[1]);
 #pragma unroll
         for (int pl = 0; pl < XP; ++pl)
 #pragma unroll
@@ -2482,16 +2495,19 @@ __device__ __attribute__((always_inline)) inline void any_run(const MapArgs& a, 
         if (ct & 1) __builtin_amdgcn_sched_barrier(0);
       }
     } else {
-      typename AnyIO<IO>::Frag wf[2][WT];  // [row tile][term]
+      // [row tile][term], and for a key's scaled second term the first over that scale.
+      constexpr bool LOW = IS_K && AnyIO<IO>::kLowScale != 1.f;
+      typename AnyIO<IO>::Frag wf[2][WT + LOW];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const f32x4 w0 = wr[part][t][0], w1 = wr[part][t][1];
         const float w[8] = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3]};
         uint32_t h[WT][4];
-        any_split<IO>(w, h);
+        any_split<IO, false>(w, h);
 #pragma unroll
         for (int p = 0; p < WT; ++p)
           wf[t][p] = __builtin_bit_cast(typename AnyIO<IO>::Frag, make_uint4(h[p][0], h[p][1], h[p][2], h[p][3]));
+        if constexpr (LOW) wf[t][WT] = wf[t][0] * static_cast<_Float16>(1.f / AnyIO<IO>::kLowScale);
       }
       // The next column tile's inputs are read during this one's products
       // (where its three planes leave the registers for it: not with CT 8).
@@ -2509,7 +2525,7 @@ __device__ __attribute__((always_inline)) inline void any_run(const MapArgs& a, 
         if (NB == 1 && ct > 0) read_x(ct);
         for_products<XP, WT>([&](int i, int j) {
 #pragma unroll
-          for (int t = 0; t < 2; ++t) acc[t][ct] = AnyIO<IO>::mul(wf[t][j], xf[ct % NB][i], acc[t][ct]);
+          for (int t = 0; t < 2; ++t) acc[t][ct] = AnyIO<IO>::mul(wf[t][LOW && i > 0 ? WT : j], xf[ct % NB][i], acc[t][ct]);
         });
         __builtin_amdgcn_sched_barrier(0);
       }

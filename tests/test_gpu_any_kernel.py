@@ -2,9 +2,10 @@
 
 Tiles hold 64 or 128 tokens, column tiles 16; waves own 16 output pairs and
 chunks 32 input pairs, so the head dims here leave every kind of remainder
-(half sizes 3, 40, 48, 64, 80, 128, 160, 256). The split operands keep at
-least 22 bits, so the mapped rows are held to 2^-18 of their summands'
-magnitude where rounding to the pool's type does not decide.
+(half sizes 3, 40, 48, 64, 80, 128, 160, 256). The split operands keep 22
+to 24 bits (fp16 keys below 2^-16 fewer: an absolute 2^-38), so the
+mapped rows are held to 2^-18 of their summands' magnitude where rounding to
+the pool's type does not decide.
 """
 
 from __future__ import annotations
@@ -57,6 +58,34 @@ def test_tiles_and_remainders_match_oracle(dim, dtype, support, tokens):
     # (A page of one token is too small a sample for the share within 1 ulp.)
     ot.check_mapped(out, _reference(spec, page, 11), bound, abs_factor=2.0 ** -18,
                     min_within_ulp=0.999 if tokens > 16 else 0.99)
+
+
+@pytest.mark.parametrize("dim", [64, 128, 256])
+@pytest.mark.parametrize("scale,mixed", [(1.0, False), (1e-2, False), (1e-3, False), (1e-4, False), (1.0, True),
+                                         (1e-2, True)])
+def test_small_half_precision_keys_keep_their_bits(dim, scale, mixed):
+    """fp16 keys far below 1, mapped up by large weights, alone or as quiet
+    channels (down to 2^-8 of the loudest, with weights to match).
+
+    fp32 multiply-adds leave a relative error of 2e-7, an ulp is 2^-11 to
+    2^-10: at most about 0.01% of the elements (those near a cancellation) may
+    lie two ulps apart, and no summand more than 2^-20 of the bound (32-bit
+    sums of up to 256 terms: 256 2^-24 at worst, their root for random signs).
+    """
+    print(f"small fp16 keys D={dim} scale={scale} mixed={mixed}", flush=True)
+    g, spec, _ = _mapper(dim, torch.float16, 1)
+    channel = torch.full((dim // 2,), scale)
+    if mixed:
+        channel = channel * 2.0 ** torch.randint(-8, 1, (dim // 2,), generator=g)
+    channel = channel.repeat(2)  # RoPE partners share their scale
+    spec["k_weight"] = spec["k_weight"] / channel[:, None] * (100 * scale if scale < 1 else 1)
+    mapper = HeadwiseMapper.from_assignment(**spec, source_rope_theta=1e4, target_rope_theta=1e6, dtype=torch.float16,
+                                            device="cuda", max_positions=1024)
+    page = (torch.randn(2, 5, 160, 2, dim, generator=g) * channel).to(torch.float16)
+    out = mapper.map_page(page.cuda(), position_start=11, output_device="cuda")
+    ref = _reference(spec, page, 11)
+    bound = ot.magnitude_bound(page, spec, position_start=11, source_theta=1e4, target_thetas=1e6)
+    ot.check_mapped(out[:1], ref[:1], bound[:1], abs_factor=2.0 ** -20, min_within_ulp=0.9995)
 
 
 @pytest.mark.parametrize("dim,dtype", [(256, torch.bfloat16), (128, torch.float16), (128, torch.float32)])

@@ -2099,8 +2099,11 @@ __global__ void pack_weights_kernel(const float* __restrict__ w, const float* __
 // bf16 terms: 1.658142e-3), at D 128 fp32 2.11e-7 with those, 1.57e-7 here.
 // An output that is not finite (an infinity or NaN in its source row, or an
 // fp16 key of 2^14 or more, whose scaled first term is infinite) is
-// computed again term by term in fp32, because an infinity times the terms of
-// a weight need not keep its sign.
+// computed again with fp32 products, because an infinity times the terms of a
+// weight need not keep its sign. The wave repeats the whole column tile on the
+// fp32 matrix instructions: D 256 bf16, 2048 tokens, 0.59 ms with no such row,
+// 0.76 with 2 of them, 2.3 with 5%, 2.7 with all (one lane per token at a
+// time, as first written: 3.6, 43 and 66 ms; plain fp32 multiply-adds 16.5).
 //
 // Fragment layout (lane l: row or column l % 16, group g = l / 16): a part's
 // 32 dims are one MFMA k-step with lane group g holding dims 8g .. 8g + 7 (in
@@ -2126,15 +2129,6 @@ __host__ __device__ inline int any_chunks(int D) { return (D / 2 + 31) / 32; }  
 __host__ __device__ inline int any_groups(int D) { return (D / 2 + 15) / 16; }   // 16-pair output groups
 // 16-byte units of one (chunk, part, output group): two row tiles x two 4-dim halves x 64 lanes.
 constexpr int kAnyFragU4 = 2 * 2 * kWave;
-// Float offset of W[member dim i][output o] of a job in the packed maps.
-__host__ __device__ inline int64_t any_w_offset(int D, int member, int i, int o) {
-  const int half = D / 2, part = i >= half, jp = part ? i - half : i;
-  const int tile = o >= half, op = tile ? o - half : o;
-  const int64_t stage = (static_cast<int64_t>(member) * any_chunks(D) + jp / 32) * 2 + part;
-  const int lane = (op & 15) + 16 * ((jp & 31) >> 3), e = jp & 7;
-  return (((stage * any_groups(D) + op / 16) * 2 + tile) * 2 + (e >> 2)) * (kWave * 4) + lane * 4 + (e & 3);
-}
-
 template <typename IO>
 struct AnyIO;
 template <>
@@ -2407,6 +2401,21 @@ __device__ __attribute__((always_inline)) inline void any_run(const MapArgs& a, 
       if constexpr (IS_K) utab = (thetas(job_then) & 0xff) * a.theta_stride;
     }
   };
+  // Element e of both parts' raw words; a pair un-rotated.
+  auto unpack_pair = [](const uint32_t (&w)[2][RW], int e, float& x1, float& x2) __attribute__((always_inline)) {
+    if constexpr (F32) {
+      x1 = __uint_as_float(w[0][e]);
+      x2 = __uint_as_float(w[1][e]);
+    } else {
+      x1 = e & 1 ? AnyIO<IO>::hi(w[0][e >> 1]) : AnyIO<IO>::lo(w[0][e >> 1]);
+      x2 = e & 1 ? AnyIO<IO>::hi(w[1][e >> 1]) : AnyIO<IO>::lo(w[1][e >> 1]);
+    }
+  };
+  auto unrotate = [](float c, float s, float& x1, float& x2) __attribute__((always_inline)) {
+    const float k1 = __builtin_fmaf(x1, c, x2 * s), k2 = __builtin_fmaf(x2, c, -(x1 * s));
+    x1 = k1;
+    x2 = k2;
+  };
   // Un-rotate and split the raw chunk into X buffer `x`.
   auto convert = [&](uint4* x) __attribute__((always_inline)) {
     auto put = [&](int plane, int part, uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3) __attribute__((always_inline)) {
@@ -2422,17 +2431,8 @@ __device__ __attribute__((always_inline)) inline void any_run(const MapArgs& a, 
       float k1[8], k2[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        float x1, x2;
-        if constexpr (F32) {
-          x1 = __uint_as_float(raw[0][e]);
-          x2 = __uint_as_float(raw[1][e]);
-        } else {
-          x1 = e & 1 ? AnyIO<IO>::hi(raw[0][e >> 1]) : AnyIO<IO>::lo(raw[0][e >> 1]);
-          x2 = e & 1 ? AnyIO<IO>::hi(raw[1][e >> 1]) : AnyIO<IO>::lo(raw[1][e >> 1]);
-        }
-        const float c = uc[e >> 2][e & 3], s = us[e >> 2][e & 3];
-        k1[e] = __builtin_fmaf(x1, c, x2 * s);
-        k2[e] = __builtin_fmaf(x2, c, -(x1 * s));
+        unpack_pair(raw, e, k1[e], k2[e]);
+        unrotate(uc[e >> 2][e & 3], us[e >> 2][e & 3], k1[e], k2[e]);
         k1[e] *= AnyIO<IO>::kKeyScale;
         k2[e] *= AnyIO<IO>::kKeyScale;
       }
@@ -2559,39 +2559,52 @@ __device__ __attribute__((always_inline)) inline void any_run(const MapArgs& a, 
     }
   };
 
-  // y of output pairs jo + i for one token, term by term in fp32 (rare: only
-  // where the split sum is not finite).
-  auto slow = [&](int tk, int jo, const float (&inv)[2][4], float (&y)[2][4]) __attribute__((always_inline)) {
-    const int job = cur.job;
-    const int64_t ro = row_of(a.src, tk) * a.src.row_stride_b;
-    const int p = position_of(a, tk);
-    const int64_t ut = (thetas(job) & 0xff) * a.theta_stride;
+  // The sums of column tile ct again, of fp32 products (rare: only where the
+  // split sum of one of its tokens is not finite). The lane's eight dims of
+  // each part are gathered anew; W's fragments are the main loop's. The job
+  // and D are hidden, so that none of this takes scalar registers from the
+  // main loop (300 of them spill to lanes, and 60 more cost it 4%).
+  auto sum_again = [&](const AnyRows<TT>& r, int ct, f32x4 (&sum)[2]) __attribute__((always_inline)) {
+    const int t = mg * 16 * CT + 16 * ct + col;
+    const int job = hide(cur.job), d = hide(D), half_d = d >> 1, nq = any_chunks(d), nc = S * nq;
+    const int64_t stage_b = static_cast<int64_t>(any_groups(d)) * kAnyFragU4 * 16;
+    const int64_t so = r.src[t];
+    const int64_t ut = (thetas(job) & 0xff) * a.theta_stride + static_cast<int64_t>(r.pos[t]) * (32 * nq) + 8 * g;
+    sum[0] = sum[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    int k = 0, q = 0;  // chunk c: member, 32-pair chunk of it
+#pragma unroll 1
+    for (int c = 0; c < nc; ++c) {
+      const int j = 32 * q + 8 * g;
+      const int valid = min(max(half_d - j, 0), 8);
+      const bool ok = so >= 0 && valid > 0;
+      gcptr p = ok ? head_base(job, k) + so + j * eb : zrow;
+      uint32_t rw[2][RW];
+      any_load8<IO, WIDE>(p, ok ? valid : 0, rw[0]);
+      any_load8<IO, WIDE>(ok ? p + half_d * eb : zrow, ok ? valid : 0, rw[1]);
+      float x[2][8];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+      for (int e = 0; e < 8; ++e) unpack_pair(rw, e, x[0][e], x[1][e]);
+      if constexpr (IS_K) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) y[t][i] = 0.f;
-    for (int k = 0; k < S; ++k) {
-      const int pr = cload(a.pairs + static_cast<int64_t>(job) * S + k);
-      gcptr sb = layer_base(a.src, kind, pr & 0xffff) + static_cast<int64_t>((pr >> 16) - a.src.head_offset) * D * eb;
-      const CB_GLOBAL IO* row = reinterpret_cast<const CB_GLOBAL IO*>(sb + ro);
-      const CB_GLOBAL float* w = gtab(reinterpret_cast<const float*>(a.w)) +
-                                 static_cast<int64_t>(job) * NC * 2 * NG * kAnyFragU4 * 4;
-      for (int d = 0; d < D; ++d) {
-        const int j = d < half ? d : d - half;
-        const float x1 = AnyIO<IO>::get(row + j), x2 = AnyIO<IO>::get(row + j + half);
-        float x = d < half ? x1 : x2;
-        if (IS_K) {
-          const int64_t at = ut + static_cast<int64_t>(p) * HP + j;
-          const float c = gtab(a.ucos_tab)[at], s = gtab(a.usin_tab)[at];
-          x = d < half ? __builtin_fmaf(x1, c, x2 * s) : __builtin_fmaf(x2, c, -(x1 * s));
-        }
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            y[t][i] = __builtin_fmaf(x, w[any_w_offset(D, k, d, t * half + min(jo + i, half - 1))] *
-                                                (AnyIO<IO>::kScaled ? inv[t][i] : 1.f), y[t][i]);
+        for (int e = 0; e < 8; ++e)
+          unrotate(gtab(a.ucos_tab)[ut + 32 * q + e], gtab(a.usin_tab)[ut + 32 * q + e], x[0][e], x[1][e]);
       }
+#pragma unroll
+      for (int part = 0; part < 2; ++part) {
+        gcptr wp = as_global(a.w) + (static_cast<int64_t>(job) * nc * 2 + 2 * c + part) * stage_b +
+                   (min(ng, any_groups(d) - 1) * (kAnyFragU4 * 16) + lane * 16);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 w0 = gload<f32x4>(wp + h * (kWave * 16)), w1 = gload<f32x4>(wp + (2 + h) * (kWave * 16));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            sum[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(w0[e], x[part][4 * h + e], sum[0], 0, 0, 0);
+            sum[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[e], x[part][4 * h + e], sum[1], 0, 0, 0);
+          }
+        }
+      }
+      q = q + 1 == nq ? 0 : q + 1;
+      k += q == 0;
     }
   };
 
@@ -2742,16 +2755,23 @@ __device__ __attribute__((always_inline)) inline void any_run(const MapArgs& a, 
       }
     }
     if (!F32 && __builtin_amdgcn_ballot_w64(again != 0)) {
+#pragma unroll 1
       for (int ct = 0; ct < nct; ++ct) {
-        if (!(again >> ct & 1)) continue;
-        const int t = mg * 16 * CT + 16 * ct + col;
-        if (tab[rb].tgt[t] < 0) continue;
-        float y[2][4];
-        const int js = hide(jo_);
-        slow(cur.lo + t, js, inv, y);
-        f32x4 c = {}, sn = {};
+        const bool mine = again >> ct & 1;
+        if (!__builtin_amdgcn_ballot_w64(mine)) continue;
+        const int t = mg * 16 * CT + 16 * ct + col, js = hide(jo_);
+        f32x4 sum[2], c = {}, sn = {};
+        sum_again(tab[rb], ct, sum);
         if constexpr (IS_K) rotation(tab[rb], t, js, c, sn);
-        finish(tab[rb], stage, t, js, bs, c, sn, y, true);
+        float y[2][4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            y[h][i] = sum[h][i];
+            if constexpr (AnyIO<IO>::kScaled) y[h][i] *= inv[h][i];
+          }
+        finish(tab[rb], stage, t, js, bs, c, sn, y, mine);
       }
     }
     if constexpr (STAGED) {
@@ -2801,8 +2821,8 @@ __global__ __launch_bounds__(NW * kWave, 2) void map_install_any_kernel(MapArgs 
   }
 }
 
-// Plan data of the general kernel: W in fragment order (any_w_offset, padded
-// entries zero), for fp16 with every output dim scaled by the power of two
+// Plan data of the general kernel: W in fragment order (padded entries
+// zero), for fp16 with every output dim scaled by the power of two
 // that brings its largest weight into [2^13, 2^14), the inverse scales, and
 // the bias, in sorted job order. Grid: (jobs, shares of a job's entries).
 __global__ __launch_bounds__(256) void pack_any_kernel(const float* __restrict__ w, const float* __restrict__ bias,

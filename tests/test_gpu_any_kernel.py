@@ -132,3 +132,44 @@ def test_infinities_and_nans_come_out_as_in_fp32(dim, dtype):
     assert torch.equal(torch.isnan(out[1]), torch.isnan(ref[1]))
     assert torch.equal(out[1][torch.isinf(ref[1])], ref[1][torch.isinf(ref[1])])
     assert torch.equal(torch.isfinite(out), torch.isfinite(ref))
+
+
+@pytest.mark.parametrize("dim,support", [(128, 1), (80, 2), (256, 1)])
+def test_recomputed_tiles_match_oracle(dim, support):
+    """fp16 keys of 2^14 and more (finite, but not as scaled terms) take the
+    recompute beside tokens that do not; outputs stay in range by small maps."""
+    print(f"large fp16 keys D={dim} s={support}", flush=True)
+    g, spec, _ = _mapper(dim, torch.float16, support)
+    spec["k_weight"] = spec["k_weight"] * 0.1
+    mapper = HeadwiseMapper.from_assignment(**spec, source_rope_theta=1e4, target_rope_theta=1e6, dtype=torch.float16,
+                                            device="cuda", max_positions=1024)
+    page = torch.randn(2, 5, 150, 2, dim, generator=g)
+    page[0, :, [0, 5, 40, 41, 77, 149]] *= 15000
+    page = page.clamp(-65504, 65504).to(torch.float16)
+    assert bool((page[0].abs() > 2 ** 14).any())
+    out = mapper.map_page(page.cuda(), position_start=11, output_device="cuda")
+    bound = ot.magnitude_bound(page, spec, position_start=11, source_theta=1e4, target_thetas=1e6)
+    ot.check_mapped(out, _reference(spec, page, 11), bound, abs_factor=2.0 ** -18, min_within_ulp=0.999)
+
+
+@pytest.mark.parametrize("dim,dtype", [(256, torch.bfloat16), (128, torch.float16)])
+def test_rows_that_are_not_finite_cost_a_few_passes(dim, dtype):
+    """A page of NaN rows against a finite one: one fp32 pass beside the split
+    one (3 to 4.5 times the time here), not the 25 to 110 times that a
+    term-by-term recompute per lane took."""
+    print(f"time of NaN rows D={dim} {dtype}", flush=True)
+    g, _, mapper = _mapper(dim, dtype, 1, lt=24, ht=8)
+    page = torch.randn(2, 5, 1024, 2, dim, generator=g).to(dtype).cuda()
+    nans = torch.full_like(page, float("nan"))
+    out = torch.empty(2, 24, 1024, 8, dim, dtype=dtype, device="cuda")
+    times = {}
+    for name, rows in (("finite", page), ("nan", nans), ("finite", page), ("nan", nans)):  # the first pair warms up
+        start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(5):
+            mapper.map_page(rows, position_start=0, output_device="cuda", output=out)
+        stop.record()
+        torch.cuda.synchronize()
+        times[name] = start.elapsed_time(stop)
+    assert bool(torch.isnan(out).all())
+    assert times["nan"] <= 10 * times["finite"], times

@@ -2143,7 +2143,10 @@ struct AnyIO<uint16_t> {  // bf16
   static __device__ uint32_t pack(float a, float b) { return pack_bf16(a, b); }
   static __device__ float lo(uint32_t w) { return lo_bf(w); }
   static __device__ float hi(uint32_t w) { return hi_bf(w); }
-  static __device__ float rest(float v, float term, float) { return v - term; }
+  static __device__ __attribute__((always_inline)) void rest(float& a, float& b, uint32_t terms, float) {
+    a = a - lo(terms);
+    b = b - hi(terms);
+  }
   static __device__ f32x4 mul(const Frag& a, const Frag& b, const f32x4& c) { return mfma(a, b, c); }
 };
 template <>
@@ -2161,8 +2164,16 @@ struct AnyIO<_Float16> {
   }
   static __device__ float lo(uint32_t w) { return static_cast<float>(__builtin_bit_cast(f16x2, w)[0]); }
   static __device__ float hi(uint32_t w) { return static_cast<float>(__builtin_bit_cast(f16x2, w)[1]); }
-  // (v - term) * low, exact: one instruction that converts the term, one more for a low other than 1.
-  static __device__ float rest(float v, float term, float low) { return __builtin_fmaf(-term, low, v * low); }
+  // What a packed pair of terms leaves of a and b, times `low` (a power of two;
+  // exact). The mixed-precision multiply-add converts the term on its way,
+  // which the compiler does not find (40x2 -> 64x2 at D 128, 1000 tokens: 68.4
+  // -> 62.9 us).
+  static __device__ __attribute__((always_inline)) void rest(float& a, float& b, uint32_t terms, float low) {
+    a *= low;
+    b *= low;
+    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel_hi:[1,0,0]" : "+v"(a) : "v"(terms), "s"(-low));
+    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(b) : "v"(terms), "s"(-low));
+  }
   static __device__ f32x4 mul(const Frag& a, const Frag& b, const f32x4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
@@ -2188,8 +2199,7 @@ __device__ __attribute__((always_inline)) inline void any_split(const float (&v)
 #pragma unroll
     for (int t = 0; t < AnyIO<IO>::kTerms; ++t) {
       h[t][e] = AnyIO<IO>::pack(a, b);
-      a = AnyIO<IO>::rest(a, AnyIO<IO>::lo(h[t][e]), low);
-      b = AnyIO<IO>::rest(b, AnyIO<IO>::hi(h[t][e]), low);
+      if (t + 1 < AnyIO<IO>::kTerms) AnyIO<IO>::rest(a, b, h[t][e], low);
     }
   }
 }

@@ -351,13 +351,13 @@ def sampled_parity(h, sh, label: str) -> dict:
     return out
 
 
-KERNEL_SOURCE = ROOT / "cachebridge_amd" / "csrc" / "cb_handoff.hip"
+KERNEL_SOURCES = [ROOT / "cachebridge_amd" / "csrc" / name for name in ("cb_handoff.hip", "cb_items.h")]
 
 
 def kernel_source_sha16() -> str:
     import hashlib
 
-    return hashlib.sha256(KERNEL_SOURCE.read_bytes()).hexdigest()[:16]
+    return hashlib.sha256(b"".join(p.read_bytes() for p in KERNEL_SOURCES)).hexdigest()[:16]
 
 
 def profiled_traffic(kernel: str, workload: str) -> tuple[int | None, str]:

@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "../../include/cachebridge_hip.h"
+#include "cb_items.h"
 
 namespace {
 
@@ -1304,7 +1305,6 @@ constexpr int kVmcnt0 = 0x0f70;
 constexpr int kVmcnt2 = 0x0f72;
 constexpr int kVmcnt6 = 0x0f76;
 
-constexpr int kSupTile = 256;                  // tokens per item
 constexpr int kSupWaves = 8;
 constexpr int kSupThreads = kSupWaves * kWave;
 constexpr int kSupStageU4 = 4 * 2 * 2 * kWave;  // uint4 per stage (16 KB)
@@ -1356,13 +1356,7 @@ __global__ void pack_support_kernel(const float* __restrict__ w, const float* __
   }
 }
 
-// Items of the support kernel: XCD x takes units x, x + 8, ... of each class
-// (the plan orders the units so that these are a run of adjacent keys jobs
-// and a run of adjacent values jobs in the sorted job order, whose support
-// lists share source layers) and runs them in groups of kSupJobGroup jobs,
-// the group's jobs interleaved per token chunk, so that the items an XCD
-// runs at one time read overlapping source rows and share its L2.
-constexpr int kSupJobGroup = 16;
+// The items of one XCD in turn (support_list_item).
 struct SupItems {
   int x, nwg;
   int64_t next;  // position in XCD x's item list
@@ -1372,26 +1366,10 @@ struct SupItems {
   };
 
   __device__ __attribute__((always_inline)) bool get(const MapArgs& a, SupItems::Item& it) const {
-    int64_t p = next;
-    for (int c = 0; c < a.ncls; ++c) {
-      const int nj = a.cls_unit_end[c] - a.cls_unit_begin[c];
-      const int mine = nj > x ? (nj - x + 7) / 8 : 0;
-      const int nch = a.cls_nchunks[c];
-      const int64_t count = static_cast<int64_t>(mine) * nch;
-      if (p < count) {
-        const int64_t gsz = static_cast<int64_t>(kSupJobGroup) * nch;
-        const int g = static_cast<int>(p / gsz);
-        const int r = static_cast<int>(p - g * gsz);
-        const int gj = min(kSupJobGroup, mine - g * kSupJobGroup);
-        const int ch = r / gj, jl = g * kSupJobGroup + (r - ch * gj);
-        it.job = cload(a.unit_job + a.cls_unit_begin[c] + x + 8 * jl);
-        it.lo = a.cls_tok_first[c] + ch * kSupTile;
-        it.hi = min(it.lo + kSupTile, a.cls_tok_first[c] + a.cls_tok_count[c]);
-        return true;
-      }
-      p -= count;
-    }
-    return false;
+    int unit;
+    if (!support_list_item(a, x, next, &unit, &it.lo, &it.hi)) return false;
+    it.job = cload(a.unit_job + unit);
+    return true;
   }
 };
 
@@ -2263,7 +2241,7 @@ struct AnySegment {
 __device__ inline bool any_segment(const MapArgs& a, int x, int seg, AnySegment* g) {
   const int c = seg >> 1;
   if (c >= a.ncls) return false;
-  g->nch = a.cls_tok_count[c] > 0 ? a.cls_nchunks[c] : 0;
+  g->nch = a.cls_nchunks[c];
   g->u0 = seg & 1 ? a.cls_val_begin[c] : a.cls_unit_begin[c];
   g->nu = (seg & 1 ? a.cls_unit_end[c] : a.cls_val_begin[c]) - g->u0;
   g->first = a.cls_tok_first[c];
@@ -3999,14 +3977,11 @@ int launch_map(const cb_plan* p, StreamArgs& a, const int64_t* first, const int6
   a.ncls = p->num_windows;
   for (int c = 0; c < p->num_windows; ++c) {
     if (first[c] + count[c] > INT32_MAX) return fail(CB_EINVAL, "launch too large");
-    const int64_t nch = (count[c] + chunk - 1) / chunk;
+    const int64_t nch = set_class_tokens(a, c, first[c], count[c], chunk);
     a.cls_unit_begin[c] = p->cls_unit_begin[c];
     a.cls_unit_end[c] = p->cls_unit_end[c];
     a.cls_val_begin[c] = p->cls_val_begin[c];
     a.cls_job_begin[c] = p->cls_job_begin[c];
-    a.cls_tok_first[c] = static_cast<int32_t>(first[c]);
-    a.cls_tok_count[c] = static_cast<int32_t>(count[c]);
-    a.cls_nchunks[c] = static_cast<int32_t>(std::max<int64_t>(nch, 1));
     a.cls_item_begin[c] = static_cast<int32_t>(items);
     items += static_cast<int64_t>(brief ? p->cls_jobs[c] : p->cls_unit_end[c] - p->cls_unit_begin[c]) * nch;
     n_total = std::max(n_total, first[c] + count[c]);

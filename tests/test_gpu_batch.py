@@ -100,6 +100,31 @@ def _some_layer_keeps_last_token(sh, sp):
     return any(w is None or last >= prefix - (w - 1) for w in (sh.windows or [None]))
 
 
+@pytest.mark.parametrize("windows", [[40, 300, 40, 300, 90], [300, 40, None, 40, 300]])
+@pytest.mark.parametrize("tokens", [100, 200, 600])
+def test_support_classes_without_tokens(windows, tokens):
+    """Early blocks of a long prefix at support 4: windows that have not opened
+    keep no token, alone or before and after classes that do."""
+    print(f"support batch windows={windows} tokens={tokens}", flush=True)
+    sh = synthetic.Shape("closed_windows", 9, 3, 5, 3, 128, 2 * tokens, torch.bfloat16, [], target_theta=1e6,
+                         windows=windows, head_map="identity", target_pages=256, seed=43, support=4)
+    h = synthetic.make_handoff(sh, fill_target="zeros")
+    pages = h.target_pool.pages
+    for prefixes in ([tokens + 45, tokens + 100], [tokens + 120, 0], [4096, 4096]):
+        h.target_pool.k_data.zero_()
+        h.target_pool.v_data.zero_()
+        spans, bt = _batch([tokens, tokens], [0, 0], prefixes, pages, seed=13)
+        check_batch_equals_single(h, spans, bt.to(h.target_pool.device))
+        kept = torch.zeros(5, h.target_pool.size, dtype=torch.bool)
+        for sp, prefix in zip(spans, prefixes):
+            for layer, window in enumerate(windows):
+                first = 0 if window is None else min(tokens, max(0, (prefix or tokens) - (window - 1)))
+                u = torch.arange(first, tokens) + sp.target_offset
+                kept[layer, bt[u // 16].long() * 16 + u % 16] = True
+        written = (h.target_pool.v_data != 0).flatten(2).any(2).cpu()
+        assert torch.equal(written, kept), prefixes
+
+
 def test_batch_flags_out_of_range_rows_and_skips_them():
     sh = _shape("tp4", 96, 2)
     h = synthetic.make_handoff(sh, target_pages=16, fill_target="zeros")

@@ -2241,7 +2241,7 @@ struct AnySegment {
 __device__ inline bool any_segment(const MapArgs& a, int x, int seg, AnySegment* g) {
   const int c = seg >> 1;
   if (c >= a.ncls) return false;
-  g->nch = a.cls_nchunks[c];
+  g->nch = a.cls_tok_count[c] > 0 ? a.cls_nchunks[c] : 0;
   g->u0 = seg & 1 ? a.cls_val_begin[c] : a.cls_unit_begin[c];
   g->nu = (seg & 1 ? a.cls_unit_end[c] : a.cls_val_begin[c]) - g->u0;
   g->first = a.cls_tok_first[c];

@@ -49,6 +49,57 @@ def test_short_rows_equal_streaming_rows(dim, dtype, tokens):
     assert bool((short[0] != 0.25).any())
 
 
+@pytest.mark.parametrize("tokens,prefix,windows", [
+    (900, 1300, [None, 40, 300, 600]),    # two closed windows at the end, one open in between
+    (900, 1100, [None, 40, 300, 150]),    # two closed ones between others
+    (900, 940, [500, 40, 300, 150]),      # one closed at the start
+    (900, 5000, [None, 40, 300, 600]),
+])
+def test_streaming_line_steps_over_closed_windows(tokens, prefix, windows):
+    """Early blocks of a prefix at the streaming kernel: the rows are the short
+    kernel's wherever the classes without tokens lie."""
+    print(f"closed windows={windows} prefix={prefix}", flush=True)
+    lt = 12
+    sh = synthetic.Shape("closed", 6, 3, lt, 3, 64, tokens, torch.bfloat16, [0, 2, 3, 5], source_theta=1e6,
+                         target_theta=[1e6 if windows[l % 4] is None else 1e4 for l in range(lt)],
+                         windows=[windows[l % 4] for l in range(lt)], target_pages=tokens // 16 + 2, seed=39)
+    h = synthetic.make_handoff(sh, fill_target="zeros")
+
+    def run(cap):
+        map_install_block(h.mapper, h.source_pool, h.source_slots, h.target_pool, start=0, stop=tokens,
+                          block_table=h.block_table, page_size=16, prefix_length=prefix, tokens_per_workgroup=cap)
+
+    short = _pools(h, lambda: run(0))
+    groups = h.mapper.plan.last_split()[1]
+    stream = _pools(h, lambda: run(16))
+    assert h.mapper.plan.last_split()[1] != groups
+    assert torch.equal(short[0], stream[0]) and torch.equal(short[1], stream[1])
+    assert bool((stream[1] != 0.25).any())
+
+
+def test_closed_windows_cost_next_to_nothing():
+    """The launch of a target whose windows have not opened against one of its
+    global layers alone (10 of 62): about the same work. Walking the 832 units
+    without tokens had taken 5 to 10 times as long."""
+    print("time of closed windows", flush=True)
+    times = {}
+    for lt, windows in ((62, [None if l % 6 == 5 else 1024 for l in range(62)]), (10, None)):
+        sh = synthetic.Shape("closed", 6, 4, lt, 16, 64, 1500, torch.bfloat16, [0, 2, 3, 5], target_theta=1e6,
+                             windows=windows, target_pages=96, seed=40)
+        h = synthetic.make_handoff(sh, fill_target="zeros")
+        for _ in range(2):  # the first turn warms up
+            start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            torch.cuda._sleep(2_000_000)
+            start.record()
+            for _ in range(20):
+                map_install_block(h.mapper, h.source_pool, h.source_slots, h.target_pool, start=0, stop=1500,
+                                  block_table=h.block_table, page_size=16, prefix_length=9000)
+            stop.record()
+            torch.cuda.synchronize()
+            times[lt] = start.elapsed_time(stop)
+    assert times[62] <= 2 * times[10], times
+
+
 def test_short_batch_equals_per_request_rows():
     """Ragged requests (one empty, one inside its prefix) in one short launch."""
     print("short batch", flush=True)

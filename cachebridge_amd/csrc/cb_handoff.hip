@@ -3910,18 +3910,36 @@ void split_cost_line(const cb_plan* p, StreamArgs* a, bool allow_pool) {
 // tokens 66 / 61; 48 fp32 jobs at D 64, 256 tokens 10.3 / 6.5, 1000 tokens
 // 14.1 / 11.3. Chunks keep two workgroups per CU busy: at 256 jobs, 128 tokens
 // take 11.6 us in two chunks and 12.4 in one, 256 tokens 18.0 in two and 20.0
-// in four.
+// in four. bf16 at D 64 and batches follow the same line: 256 jobs at D 64, 64
+// tokens 8.7 / 5.9, 320 tokens 15.1 / 11.7; batches of 3 and 6 requests of
+// about 70 tokens 21.4 / 20.2, 32.7 / 32.3.
+//
+// Window classes of unequal token counts: a workgroup that maps one of few
+// long jobs whole outlasts all others (62 layers with every sixth one global,
+// windows of 64: 400 tokens 66 / 119, and 2000 tokens at 256 jobs 26 / 80), so
+// jobs go to workgroups round by round, as long as these are not many more
+// than the jobs or fit the chip at once. Streaming / short with 64-token
+// chunks, by rounds per job: 1984 jobs, 1.2 rounds 54.7 / 41.0, 1.5 rounds
+// 62.4 / 56.3, 1.6 rounds 66.2 / 54.5, 2.0 rounds 66.4 / 69.8, 2.2 rounds 61.9 /
+// 70.4; 256 jobs, 376 rounds 12.8 / 10.9, 496 rounds 14.6 / 12.1, 632 rounds
+// 15.2 / 16.2, 832 rounds 16.9 / 19.5. Jobs of a class without tokens don't
+// count.
 int short_chunk(const cb_plan* p, const int64_t* count) {
-  int64_t jobs = 0, job_tokens = 0, most = 0;
+  const auto up = [](int64_t n, int64_t d) { return (n + d - 1) / d; };
+  int64_t jobs = 0, job_tokens = 0, rounds = 0, most = 0;
   for (int c = 0; c < p->num_windows; ++c) {
+    if (count[c] <= 0 || p->cls_jobs[c] == 0) continue;
     jobs += p->cls_jobs[c];
     job_tokens += p->cls_jobs[c] * count[c];
+    rounds += p->cls_jobs[c] * up(count[c], kRoundTokens);
     most = std::max(most, count[c]);
   }
-  if (job_tokens > 112 * jobs + 256 * static_cast<int64_t>(p->num_cus)) return 0;
-  const int64_t chunks = std::max<int64_t>(1, 2 * static_cast<int64_t>(p->num_cus) / std::max<int64_t>(jobs, 1));
-  const int64_t tokens = (most + chunks - 1) / chunks;
-  return static_cast<int>(std::max<int64_t>(1, (tokens + kRoundTokens - 1) / kRoundTokens) * kRoundTokens);
+  const int64_t slots = 2 * static_cast<int64_t>(p->num_cus);  // workgroups that run at one time
+  if (jobs == 0 || job_tokens > 112 * jobs + 128 * slots) return 0;
+  if (4 * most * jobs > 5 * job_tokens && most > kRoundTokens)
+    return rounds <= std::max(jobs * 7 / 4, slots) ? kRoundTokens : 0;
+  const int64_t chunks = std::max<int64_t>(1, slots / jobs);
+  return static_cast<int>(up(up(most, chunks), kRoundTokens) * kRoundTokens);
 }
 
 template <typename IO>

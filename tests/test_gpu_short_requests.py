@@ -49,6 +49,36 @@ def test_short_rows_equal_streaming_rows(dim, dtype, tokens):
     assert bool((short[0] != 0.25).any())
 
 
+@pytest.mark.parametrize("tokens,window,prefix,items", [
+    (200, 64, 0, 40 * 4 + 216),       # few long jobs: round by round
+    (400, 64, 0, 40 * 7 + 216),
+    (600, 128, 0, None),              # more rounds than the chip holds: the streaming kernel
+    (2000, 64, 0, None),
+    (600, 1024, 5000, 40 * 10),       # windows that have not opened: 12 chunks a global job fill the chip
+    (1500, 1024, 5000, 40 * 12),
+])
+def test_unequal_window_classes(tokens, window, prefix, items):
+    """Which kernel maps a request whose window classes keep unequal token
+    counts, and that its rows are the streaming kernel's."""
+    print(f"unequal classes T={tokens} window={window} prefix={prefix}", flush=True)
+    windows = [None if l % 6 == 5 else window for l in range(64)]
+    sh = synthetic.Shape("unequal", 6, 2, 64, 2, 64, tokens, torch.bfloat16, [0, 2, 3, 5], source_theta=1e6,
+                         target_theta=[1e6 if w is None else 1e4 for w in windows], windows=windows,
+                         target_pages=tokens // 16 + 2, seed=37)
+    h = synthetic.make_handoff(sh, fill_target="zeros")
+
+    def run(cap):
+        map_install_block(h.mapper, h.source_pool, h.source_slots, h.target_pool, start=0, stop=tokens,
+                          block_table=h.block_table, page_size=16, prefix_length=prefix, tokens_per_workgroup=cap)
+
+    got = _pools(h, lambda: run(0))
+    groups = h.mapper.plan.last_split()[1]
+    cus = torch.cuda.get_device_properties(0).multi_processor_count // 8 * 8
+    stream = _pools(h, lambda: run(512))
+    assert torch.equal(got[0], stream[0]) and torch.equal(got[1], stream[1])
+    assert groups == (cus if items is None else -(-items // 8) * 8), groups
+
+
 @pytest.mark.parametrize("tokens,prefix,windows", [
     (900, 1300, [None, 40, 300, 600]),    # two closed windows at the end, one open in between
     (900, 1100, [None, 40, 300, 150]),    # two closed ones between others

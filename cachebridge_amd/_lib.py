@@ -204,6 +204,11 @@ def check(rc: int) -> None:
     raise CacheBridgeHipError(message)
 
 
+# torch's own accessor of the current stream's handle; it is not a documented
+# name, so a torch without it takes the public way.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(stream: torch.cuda.Stream | None = None) -> int:
     """Raw HIP stream handle of ``stream`` (default: torch's current stream).
 
@@ -213,4 +218,6 @@ def stream_handle(stream: torch.cuda.Stream | None = None) -> int:
     """
     if stream is not None:
         return int(stream.cuda_stream)
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if _raw_stream is None:
+        return int(torch.cuda.current_stream().cuda_stream)
+    return _raw_stream(torch.cuda.current_device())

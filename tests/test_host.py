@@ -146,3 +146,17 @@ def test_request_span_defaults():
     arr = _span_array([sp, (0, 0, 0, 7, 9)])
     assert (arr[0].source_offset, arr[0].target_offset, arr[0].num_tokens) == (10, 32, 5)
     assert (arr[1].position_start, arr[1].prefix_length, arr[1].reserved) == (7, 9, 0)
+
+
+@pytest.mark.parametrize("private", [True, False])
+def test_current_stream_handle_with_and_without_torchs_private_accessor(monkeypatch, private):
+    from cachebridge_amd import _lib
+
+    class Stream:
+        cuda_stream = 0x1234
+
+    monkeypatch.setattr(_lib, "_raw_stream", (lambda device: 0x1000 + device) if private else None)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: Stream)
+    assert _lib.stream_handle() == (0x1003 if private else 0x1234)
+    assert _lib.stream_handle(Stream) == 0x1234

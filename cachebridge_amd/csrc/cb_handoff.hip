@@ -4147,9 +4147,7 @@ int launch_map(const cb_plan* p, StreamArgs& a, const int64_t* first, const int6
     if (idle) hipLaunchKernelGGL(map_install_support_kernel<true>, dim3(8 * per_xcd), dim3(kSupThreads), 0, s, base);
     else hipLaunchKernelGGL(map_install_support_kernel<false>, dim3(8 * per_xcd), dim3(kSupThreads), 0, s, base);
   } else {
-    if (D == 128 && p->ntw == 2)
-      hipLaunchKernelGGL((map_install_gen_kernel<128, uint16_t>), grid, block, 0, s, base);
-    else if (D == 64 && p->ntw == 2)
+    if (p->ntw == 2)
       hipLaunchKernelGGL((map_install_gen_kernel<64, uint16_t>), grid, block, 0, s, base);
     else
       hipLaunchKernelGGL((map_install_gen_kernel<64, float>), grid, block, 0, s, base);

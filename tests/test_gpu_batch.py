@@ -64,6 +64,31 @@ def test_batch_equals_per_request_installs(name, layers, lengths, positions, pre
     check_batch_equals_single(h, spans, bt.to(h.target_pool.device))
 
 
+def _streamed(plan):
+    """Whether the plan's last launch was the streaming kernel's: a workgroup per CU."""
+    return plan.last_split()[1] == torch.cuda.get_device_properties(0).multi_processor_count // 8 * 8
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("windows", [None, [None, 40, 300]])
+def test_batch_equals_per_request_installs_at_head_dim_64(dtype, windows):
+    """Batches long enough for the streaming kernel (shorter ones take another),
+    whose requests alone are short ones."""
+    print(f"batch D=64 {dtype} windows={windows}", flush=True)
+    lt, lengths = 12, [700, 33, 0, 1200, 16, 1500]
+    sh = synthetic.Shape("batch64", 8, 2, lt, 4, 64, sum(lengths), dtype, [],
+                         target_theta=1e6 if windows is None else [1e6 if windows[l % 3] is None else 1e4
+                                                                   for l in range(lt)],
+                         windows=windows and [windows[l % 3] for l in range(lt)], seed=51)
+    pages = sum((n + 15) // 16 for n in lengths) * 2
+    h = synthetic.make_handoff(sh, target_pages=pages, fill_target="zeros")
+    spans, bt = _batch(lengths, [0, 3, 0, 77, 0, 0], [0] * 6, pages, seed=17)
+    map_install_batch(h.mapper, h.source_pool, h.source_slots, h.target_pool, spans,
+                      block_table=bt.to(h.target_pool.device), page_size=16)
+    assert _streamed(h.mapper.plan)
+    check_batch_equals_single(h, spans, bt.to(h.target_pool.device))
+
+
 def check_batch_equals_single(h, spans, bt):
     """One batched launch over ``spans`` against one ``map_install`` per request."""
     map_install_batch(h.mapper, h.source_pool, h.source_slots, h.target_pool, spans,
@@ -125,20 +150,24 @@ def test_support_classes_without_tokens(windows, tokens):
         assert torch.equal(written, kept), prefixes
 
 
-def test_batch_flags_out_of_range_rows_and_skips_them():
-    sh = _shape("tp4", 96, 2)
-    h = synthetic.make_handoff(sh, target_pages=16, fill_target="zeros")
-    spans, bt = _batch([40, 56], [0, 0], [0, 0], 16, seed=3)
+@pytest.mark.parametrize("layers,lengths", [(2, [40, 56]), (32, [500, 400])])
+def test_batch_flags_out_of_range_rows_and_skips_them(layers, lengths):
+    """In a batch of the short kernel and in one of the streaming kernel."""
+    pages = sum((n + 15) // 16 for n in lengths) + 9
+    sh = _shape("tp4", sum(lengths), layers)
+    h = synthetic.make_handoff(sh, target_pages=pages, fill_target="zeros")
+    spans, bt = _batch(lengths, [0, 0], [0, 0], pages, seed=3)
     bt = bt.to(h.target_pool.device)
     bad = bt.clone()
     bad[1] = h.target_pool.pages + 5  # request 0's second page lies beyond the pool
     map_install_batch(h.mapper, h.source_pool, h.source_slots, h.target_pool, spans,
                       block_table=bad, page_size=16)
     assert h.mapper.plan.read_errors() & 2
+    assert _streamed(h.mapper.plan) == (layers == 32)
     good = _target_like(h.target_pool)
     # request 0 without its tokens 16..31 (the bad page): those rows are not written
     ok = [spans[0]._replace(num_tokens=16),
-          RequestSpan(spans[0].source_offset + 32, spans[0].target_offset + 32, 8, 32, 40),
+          RequestSpan(spans[0].source_offset + 32, spans[0].target_offset + 32, lengths[0] - 32, 32, lengths[0]),
           spans[1]]
     map_install_batch(h.mapper, h.source_pool, h.source_slots, good, ok, block_table=bt,
                       page_size=16)

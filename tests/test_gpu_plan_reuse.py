@@ -24,7 +24,7 @@ def _empty_like(pool):
                        device=pool.device, fill="zeros")
 
 
-@pytest.mark.parametrize("name,layers", [("tp4", 6), ("gemma", 12)])
+@pytest.mark.parametrize("name,layers", [("tp4", 32), ("gemma", 24)])
 def test_alternating_shapes_match_fresh_plans(name, layers):
     print(f"plan reuse {name} layers={layers}", flush=True)
     sh = synthetic.shape(name, tokens=3000)
@@ -34,11 +34,14 @@ def test_alternating_shapes_match_fresh_plans(name, layers):
         sh.target_theta = sh.target_theta[:layers]
     h = synthetic.make_handoff(sh, fill_target="zeros")
     shapes = [(0, 3000, 0), (0, 700, 0), (0, 3000, 0), (0, 3000, 256), (500, 2100, 0), (0, 700, 0)]
+    cus = torch.cuda.get_device_properties(0).multi_processor_count // 8 * 8
     for start, stop, tpw in shapes:
         reused = _empty_like(h.target_pool)
         map_install_block(h.mapper, h.source_pool, h.source_slots, reused, start=start, stop=stop,
                           block_table=h.block_table, page_size=sh.page_size, prefix_length=3000,
                           tokens_per_workgroup=tpw)
+        if tpw == 0:  # (with enough layers to keep the shortest of them on the kernel that keeps a split)
+            assert h.mapper.plan.last_split()[1] == cus, (start, stop)
         fresh_mapper = synthetic.make_mapper(sh, h.spec)
         fresh = _empty_like(h.target_pool)
         map_install_block(fresh_mapper, h.source_pool, h.source_slots, fresh, start=start, stop=stop,

@@ -1366,15 +1366,8 @@ struct SupItems {
   int x, nwg;
   int64_t next;  // position in XCD x's item list
 
-  struct Item {
-    int job, lo, hi;
-  };
-
-  __device__ __attribute__((always_inline)) bool get(const MapArgs& a, SupItems::Item& it) const {
-    int unit;
-    if (!support_list_item(a, x, next, &unit, &it.lo, &it.hi)) return false;
-    it.job = cload(a.unit_job + unit);
-    return true;
+  __device__ __attribute__((always_inline)) bool get(const MapArgs& a, SupItem& it) const {
+    return support_list_item(a, x, next, [&](int unit) __attribute__((always_inline)) { return cload(a.unit_job + unit); }, it);
   }
 };
 
@@ -1772,7 +1765,7 @@ __global__ __launch_bounds__(kSupThreads, 1) void map_install_support_kernel(Map
   int step = IDLE ? 2 * (items.nwg - static_cast<int>(items.next)) - 1 : items.nwg;
   uint32_t slot = 0;  // ring slot of the last stage run
   int errbits = 0;
-  SupItems::Item it;
+  SupItem it;
   for (; items.get(a, it); items.next += step, step = IDLE ? 2 * items.nwg - step : step) {
     SupLane I;
     I.job = __builtin_amdgcn_readfirstlane(it.job);

@@ -30,10 +30,14 @@ inline int64_t set_class_tokens(Args& a, int c, int64_t first, int64_t count, in
 // in the sorted job order, whose support lists share source layers) and runs
 // them in groups of kSupJobGroup jobs, the group's jobs interleaved per token
 // chunk, so that the items an XCD runs at one time read overlapping source
-// rows and share its L2. Item p of its list: a unit and a token range; false
+// rows and share its L2. Item p of its list (job_of: the job of a unit), false
 // past the end.
-template <class Args>
-CB_ITEMS_FN bool support_list_item(const Args& a, int x, int64_t p, int* unit, int* lo, int* hi) {
+struct SupItem {
+  int job, lo, hi;  // tokens [lo, hi)
+};
+
+template <class Args, class JobOf>
+CB_ITEMS_FN bool support_list_item(const Args& a, int x, int64_t p, JobOf&& job_of, SupItem& it) {
   for (int c = 0; c < a.ncls; ++c) {
     const int nj = a.cls_unit_end[c] - a.cls_unit_begin[c];
     const int mine = nj > x ? (nj - x + 7) / 8 : 0;
@@ -44,12 +48,12 @@ CB_ITEMS_FN bool support_list_item(const Args& a, int x, int64_t p, int* unit, i
       const int g = static_cast<int>(p / gsz);
       const int r = static_cast<int>(p - g * gsz);
       const int left = mine - g * kSupJobGroup;
-      const int gj = left < kSupJobGroup ? left : kSupJobGroup;
+      const int gj = kSupJobGroup < left ? kSupJobGroup : left;
       const int ch = r / gj, jl = g * kSupJobGroup + (r - ch * gj);
-      *unit = a.cls_unit_begin[c] + x + 8 * jl;
-      *lo = a.cls_tok_first[c] + ch * kSupTile;
+      it.job = job_of(a.cls_unit_begin[c] + x + 8 * jl);
+      it.lo = a.cls_tok_first[c] + ch * kSupTile;
       const int end = a.cls_tok_first[c] + a.cls_tok_count[c];
-      *hi = *lo + kSupTile < end ? *lo + kSupTile : end;
+      it.hi = it.lo + kSupTile < end ? it.lo + kSupTile : end;
       return true;
     }
     p -= count;

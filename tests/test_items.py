@@ -36,8 +36,9 @@ int main(int argc, char** argv) {
     token += t;
   }
   for (int x = 0; x < 8; ++x) {
-    int u, lo, hi;
-    for (long p = 0; support_list_item(a, x, p, &u, &lo, &hi); ++p) std::printf("%d %d %d %d\n", x, u, lo, hi);
+    SupItem it;
+    for (long p = 0; support_list_item(a, x, p, [](int unit) { return unit; }, it); ++p)
+      std::printf("%d %d %d %d\n", x, it.job, it.lo, it.hi);
   }
 }
 """

@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cstdarg>
 #include <cstdint>
@@ -384,11 +385,6 @@ struct StreamArgs : MapArgs {
   // blk_unit/sub[r + 1] (cut on the host, split_cost_line).
   int32_t blk_unit[kMaxStreamBlocks + 1];
   int32_t blk_sub[kMaxStreamBlocks + 1];
-  // Units of classes without tokens between others that have some (four
-  // classes leave room for one such run): a range steps from gap_begin to
-  // gap_end. Passing the units of a closed window one by one took 0.25 us each
-  // (62x16, every sixth layer global, 900 tokens: 252 us, 47 without).
-  int32_t gap_begin, gap_end;
 };
 
 // Job flag (meta.z): un-rotation uses the rotation table (same theta, unit norm).
@@ -995,7 +991,7 @@ __global__ __launch_bounds__(kStreamThreads) void map_install_stream_kernel(Stre
     const int c = class_of_unit(a, cur.unit);
     const int stop = cur.unit == end.unit ? end.sub : a.cls_subtiles[c];
     if (stop > cur.sub) seg(cur.unit, cur.sub, stop);
-    cur = Pos{cur.unit + 1 == a.gap_begin ? a.gap_end : cur.unit + 1, 0};
+    cur = Pos{cur.unit + 1, 0};
   }
   if (a.pool_n <= 0) return;
   // Work pool: a workgroup done with its own range claims chunks of the
@@ -3949,6 +3945,22 @@ void launch_any(int D, int64_t items, hipStream_t s, const MapArgs& a) {
   else hipLaunchKernelGGL((map_install_any_kernel<IO, 4, 2>), g, b, 0, s, a, D);
 }
 
+// Whether a line of the streaming kernel with `gap` units without tokens
+// between others is better cut into two launches. One workgroup passes the gap
+// at 0.25 us a unit, 7 of the line's weights, while the others map their
+// shares (line / num_cus each); a second launch costs 10 us and the first one's
+// uneven end. Measured at a gap of 496 units (62x16, windows of 300, 1024 and
+// none), one launch / two: 900 tokens 242 / 121 us, 2000 tokens 285 / 196, 4096
+// tokens 339 / 366.
+bool cut_at_gap(const cb_plan* p, const int64_t* count, int64_t gap) {
+  if (gap <= 40) return false;
+  int64_t line = 0;
+  for (int c = 0; c < p->num_windows; ++c)
+    for (int u = p->cls_unit_begin[c]; count[c] > 0 && u < p->cls_unit_end[c]; ++u)
+      line += kSegmentCost + p->unit_weight[u] * ((count[c] + kSubTokens - 1) / kSubTokens);
+  return 2 * 7 * gap > line / p->num_cus;
+}
+
 // Enqueue the map kernel over class token ranges [first[c], first[c] +
 // count[c]) of the launch's token space. `a` carries the two sides (and, for
 // batches, the position vector); the plan fields are filled in here.
@@ -4034,15 +4046,22 @@ int launch_map(const cb_plan* p, StreamArgs& a, const int64_t* first, const int6
       subtiles += sub;
     }
     if (subtiles == 0) return CB_OK;
-    // The line ends with the last class that has tokens.
-    static_assert(kMaxClasses <= 4, "at most one gap");
+    // Passing a unit without tokens takes a workgroup 0.25 us (62x16, every
+    // sixth layer global, the first 900 tokens of a long prefix: 252 us, 47
+    // without), so the line ends with the last class that has tokens, and one
+    // with a long gap between such classes becomes two launches. (A jump in the
+    // kernel instead slowed every short launch by 0.4 us.)
     a.num_units = 0;
-    a.gap_begin = a.gap_end = -1;
     for (int c = 0; c < p->num_windows; ++c) {
-      if (a.cls_subtiles[c] == 0 || p->cls_jobs[c] == 0) continue;
-      if (a.num_units > 0 && p->cls_unit_begin[c] != a.num_units) {
-        a.gap_begin = a.num_units;
-        a.gap_end = p->cls_unit_begin[c];
+      if (count[c] <= 0 || p->cls_jobs[c] == 0) continue;
+      if (a.num_units > 0 && cut_at_gap(p, count, p->cls_unit_begin[c] - a.num_units)) {
+        std::array<int64_t, kMaxClasses> part{};
+        std::copy(count, count + c, part.begin());
+        const int rc = launch_map(p, a, first, part.data(), tokens_per_workgroup, default_tokens, s);
+        if (rc != CB_OK) return rc;
+        part.fill(0);
+        std::copy(count + c, count + p->num_windows, part.begin() + c);
+        return launch_map(p, a, first, part.data(), tokens_per_workgroup, default_tokens, s);
       }
       a.num_units = p->cls_unit_end[c];
     }

@@ -85,24 +85,26 @@ def test_unequal_window_classes(tokens, window, prefix, items):
     (900, 940, [500, 40, 300, 150]),      # one closed at the start
     (900, 5000, [None, 40, 300, 600]),
 ])
-def test_streaming_line_steps_over_closed_windows(tokens, prefix, windows):
+@pytest.mark.parametrize("lt", [12, 64])
+def test_streaming_line_steps_over_closed_windows(lt, tokens, prefix, windows):
     """Early blocks of a prefix at the streaming kernel: the rows are the short
-    kernel's wherever the classes without tokens lie."""
-    print(f"closed windows={windows} prefix={prefix}", flush=True)
-    lt = 12
+    kernel's wherever the classes without tokens lie (at 64 layers, a gap of
+    one or two classes is long enough for a launch on either side of it)."""
+    print(f"closed windows={windows} prefix={prefix} layers={lt}", flush=True)
     sh = synthetic.Shape("closed", 6, 3, lt, 3, 64, tokens, torch.bfloat16, [0, 2, 3, 5], source_theta=1e6,
                          target_theta=[1e6 if windows[l % 4] is None else 1e4 for l in range(lt)],
                          windows=[windows[l % 4] for l in range(lt)], target_pages=tokens // 16 + 2, seed=39)
     h = synthetic.make_handoff(sh, fill_target="zeros")
 
-    def run(cap):
-        map_install_block(h.mapper, h.source_pool, h.source_slots, h.target_pool, start=0, stop=tokens,
-                          block_table=h.block_table, page_size=16, prefix_length=prefix, tokens_per_workgroup=cap)
+    def run(block, cap):
+        for start in range(0, tokens, block):
+            map_install_block(h.mapper, h.source_pool, h.source_slots, h.target_pool, start=start, stop=start + block,
+                              block_table=h.block_table, page_size=16, prefix_length=prefix, tokens_per_workgroup=cap)
 
-    short = _pools(h, lambda: run(0))
-    groups = h.mapper.plan.last_split()[1]
-    stream = _pools(h, lambda: run(16))
-    assert h.mapper.plan.last_split()[1] != groups
+    short = _pools(h, lambda: run(100, 0))
+    cus = torch.cuda.get_device_properties(0).multi_processor_count // 8 * 8
+    assert h.mapper.plan.last_split()[1] != cus  # (the streaming kernel's grid)
+    stream = _pools(h, lambda: run(tokens, 16))
     assert torch.equal(short[0], stream[0]) and torch.equal(short[1], stream[1])
     assert bool((stream[1] != 0.25).any())
 

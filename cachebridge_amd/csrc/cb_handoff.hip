@@ -2082,11 +2082,14 @@ __global__ void pack_weights_kernel(const float* __restrict__ w, const float* __
 // fp32, eight 4-dim k-steps: step e takes dim 8g + e of every group). The
 // accumulator register i of lane (col, g) is output dim 16 ng + 4g + i.
 //
-// Bound: latency and issue (MFMA 23-40% busy, HBM at 2-3 TB/s). Measured on
-// MI355X against a kernel of plain fp32 multiply-adds: 34x4 -> 48x8 at D 256
-// bf16 with windows, 2048 tokens, 16.5 -> 0.63 ms; 40x2 -> 64x2 at D 128 fp16,
-// 1000 tokens, 1.62 ms -> 69 us. What the parts cost at D 256 (removed one at
-// a time): products 16%, outputs 18%, gather and conversion 13%, W 5%.
+// Bound: latency and issue (MFMA 39% busy at D 256 bf16 with 2.0 TB/s from and
+// to memory, 12% at D 128 fp16 with 1.7). Measured on MI355X, passes back to
+// back on several cards, against a kernel of plain fp32 multiply-adds: 34x4 ->
+// 48x8 at D 256 bf16 with windows, 2048 tokens, 16.5 ms -> 570 to 650 us; 40x2
+// -> 64x2 at D 128 fp16, 1000 tokens, 1.6 ms -> 63 to 68 us. What the parts cost at
+// D 256 (removed one at a time): products 16%, outputs 18%, gather and
+// conversion 13%, W 5%. Head dims up to 6 at 16 tokens are 2 us slower than
+// that kernel was (10.5 against 8.2): one tile's chain of loads is longer here.
 // ---------------------------------------------------------------------------
 
 constexpr int kAnyTile = 32;        // granularity of tokens_per_workgroup
@@ -4248,6 +4251,11 @@ void* scratch_on(int device) {
   return g_scratch_ptr[device];
 }
 
+// Up to this many states, 64-row workgroups (two a state) all find a CU of
+// their own. Split / whole, us: 128 x 256 -> 128 x 256, 32 states 38 / 54, 128
+// states 44 / 58, 160 states 82 / 59, 256 states 89 / 63, 384 states 129 / 116;
+// 64 x 128 -> 128 x 128, 128 states 12.8 / 17.1, 160 states 18.2 / 17.9, 384
+// states 29.7 / 30.9.
 constexpr unsigned kDeltaSplitBatch = 128;
 
 // Whether delta_tile_kernel takes a transform: its dimensions, and 16-byte
@@ -4274,7 +4282,6 @@ void launch_delta_value(const DeltaArgs& a, dim3 g, hipStream_t s) {
 }
 
 void launch_delta_tile(const DeltaArgs& a, unsigned batch, hipStream_t s) {
-  // 64 rows per workgroup where the batch alone leaves CUs idle.
   if (a.kp == 64 || batch <= kDeltaSplitBatch) launch_delta_value<4>(a, dim3(batch, a.kp / 64), s);
   else launch_delta_value<8>(a, dim3(batch), s);
 }

@@ -113,7 +113,9 @@ typedef struct cb_rows {
 typedef struct cb_plan_desc {
   int32_t head_dim;  /* even, 2..512. bf16 at 64 and 128 and fp32 at 64 take the
                         MFMA kernels; every other head_dim or dtype takes the
-                        general kernel (fp32 maps, as exact as fp32 products) */
+                        general kernel (fp32 maps; errors against 64 bits no
+                        larger than fp32 multiply-adds', fp16 keys down to 1e-4
+                        included) */
   int32_t support;   /* 1..CB_MAX_SUPPORT */
   int32_t io_dtype;  /* CB_DTYPE_* */
   int32_t num_jobs;

@@ -111,8 +111,8 @@ typedef struct cb_rows {
  * support rows in pair order) plus a [head_dim] fp32 bias.
  */
 typedef struct cb_plan_desc {
-  int32_t head_dim;  /* even, 2..512. bf16 at 64 and 128 and fp32 at 64 take the
-                        MFMA kernels; every other head_dim or dtype takes the
+  int32_t head_dim;  /* even, 2..512. bf16 at 64 and 128 and fp32 at 64 have kernels
+                        of their own; every other head_dim or dtype takes the
                         general kernel (fp32 maps; errors against 64 bits no
                         larger than fp32 multiply-adds', fp16 keys down to 1e-4
                         included) */
